@@ -19,7 +19,8 @@
 //      the K/V loop needs no cross-group communication; groups merge once at the end. Block ids
 //      of the split are held one per lane and broadcast with v_readlane. Q.K uses v_dot2_f32_f16.
 //   3. attn_rows_kernel: the general version of (2) for shapes the fast path does not cover
-//      (block_size not a multiple of the tokens-per-load, or prefill tiles before the MFMA path).
+//      (block_size not a multiple of the tokens-per-load, or prefill tiles of the types and head
+//      dims that attention_prefill.hip does not take).
 //   4. attn_combine_kernel merges the fp32 split partials (m, l, acc) of split requests, one
 //      thread per (token, query head, 4 output elements); unsplit requests are written directly
 //      by (2)/(3).
@@ -896,18 +897,18 @@ void dispatch_rows_qr(const Launch& a, int qr, int base, int count, int limit_wo
   }
 }
 
-// Tile items (prefill slices) first: the MFMA tile kernel for fp16 / head_dim 64, the general
-// row kernel with 8 query vectors per pass otherwise. Row items: the fast decode kernel when
+// Tile items (prefill slices) first: the MFMA tile kernel for fp16 and bf16 with head_dim 64 or
+// 128, the general row kernel with 8 query vectors per pass otherwise. Row items: the fast decode kernel when
 // every split's load groups stay inside one block, the general kernel otherwise.
 template <typename T, int D>
 int run_items(const Launch& a, const int32_t* ph, int parts) {
   using C = RowCfg<T, D>;
   const int n_items = ph[H_N_ITEMS], n_row = ph[H_N_ROW_ITEMS];
   if ((parts & EDGERAG_ATTN_TILES) && n_items > n_row) {
-    if constexpr (__is_same(T, f16) && D == 64) {
-      if (ph[H_TILE_KIND] == 1 && prefill_tiles_supported(a.nb, a.bs)) {
-        launch_prefill_tiles_f16_d64(a, n_row, n_items - n_row,
-                                     (parts & EDGERAG_ATTN_TILES_SHARED) != 0);
+    if constexpr (!__is_same(T, float) && (D == 64 || D == 128)) {
+      if (ph[H_TILE_KIND] == 1 && prefill_tiles_supported(a.nb, a.bs, D)) {
+        launch_prefill_tiles(a, ph[H_DTYPE], D, n_row, n_items - n_row,
+                             (parts & EDGERAG_ATTN_TILES_SHARED) != 0);
       } else {
         dispatch_rows_qr<T, D>(a, 8, n_row, n_items - n_row, H_N_ITEMS);
       }
@@ -971,8 +972,9 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
                 max_blocks_per_seq);
 
   const int n_rep = n_q_heads / n_kv_heads;
-  // Prefill tiles run on MFMA for fp16 / head_dim 64: 128 virtual rows (token x head-in-group).
-  const bool mfma_tiles = dtype == EDGERAG_F16 && head_dim == 64 && n_rep <= kMfmaTileRows;
+  // Prefill tiles on MFMA: 128 virtual rows (token x head-in-group).
+  const bool mfma_tiles = prefill_tile_shape(dtype, head_dim) && n_rep <= kMfmaTileRows;
+  const bool wide_tiles = mfma_tiles && !(dtype == EDGERAG_F16 && head_dim == 64);
   const int tile_rows = mfma_tiles ? kMfmaTileRows / n_rep : kQTile;
   int64_t work = 0;       // KV token-heads the decode rows read, to size their splits
   int64_t tile_work = 0;  // tile x keys of the prefill slices, to size theirs
@@ -1104,14 +1106,19 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
   // extra split costs a partial write and a merge. Beside decode rows (overlap) the tiles run at
   // one workgroup per CU (the rows take the rest of each CU), otherwise at two: kTargetTiles / 2
   // or kTargetTiles items. (Three 512-token slices, 384 tiles, beside 24 decodes: splitting them to
-  // 768 items for the larger target measured 0.225 against 0.215 ms per step.)
+  // 768 items for the larger target measured 0.225 against 0.215 ms per step.) Batches of at most
+  // one tile per CU whose tiles hold p in 32 bits (bf16, or head_dim 128) aim at kTargetTiles / 2
+  // as well: the partials of twice the items cost more than the second workgroup per CU gains (512
+  // tokens at 3,072 keys: fp16 32/8 heads of 128 65.3 -> 62.0 us, bf16 32/32 of 64 43.3 -> 40.9;
+  // bf16 32/8 of 128, slices at 2,048 and 4,096: 139 -> 128 us).
   // A split may span at most kMaxTileBlocks blocks (the MFMA tile kernel stages its block ids).
-  const int64_t target_tiles = overlap ? kTargetTiles / 2 : kTargetTiles;
+  const int64_t target_tiles =
+      overlap || (wide_tiles && n_tiles <= kPlanCUs) ? kTargetTiles / 2 : kTargetTiles;
   const int64_t tile_split_cap =
       std::max<int64_t>(64, int64_t(kMaxTileBlocks - 1) * block_size / 64 * 64);
   const int64_t tile_share = round_up(
       std::max<int64_t>(kMinTileSplit, (tile_work + target_tiles - 1) / target_tiles), 64);
-  const int64_t tile_part = std::min(
+  int64_t tile_part = std::min(
       tile_split_cap, (EDGERAG_TILE_BALANCE || n_tiles < target_tiles)
                           ? tile_share
                           : round_up(std::max<int64_t>(max_len, 1), 64));
@@ -1120,6 +1127,36 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
     const int64_t n = std::max<int64_t>(1, (L + tile_part - 1) / tile_part);
     return std::min(tile_split_cap, round_up((std::max<int64_t>(L, 1) + n - 1) / n, 64));
   };
+
+  // Keys of a request's splits and its partial slots per (token, query head); slots 1: no partials.
+  struct RequestSplit {
+    int64_t len;
+    int n, pstride;
+  };
+  auto request_split = [&](int64_t c, int64_t L) -> RequestSplit {
+    const bool row = c * n_rep <= kMaxRowVecs;
+    // Workgroup-split rows: one item per part of the context (the waves split the part).
+    const int64_t slen = row ? (wg_rows ? wg_split_len(L) : split_len) : tile_split_len(L);
+    const int n = c == 0 ? 0 : int((L + slen - 1) / slen);
+    // Slotted row requests write partials (and get merge rows) even when not split.
+    return {slen, n, slots > 0 && row ? slots : n};
+  };
+  // The partials of the wide tiles (128 rows of head_dim 128 take 66 KB a split) fit the static
+  // scratch of edgerag_paged_attention_noalloc wherever longer splits make them fit: past it,
+  // tiles are split less. (fp16 head_dim 64 plans keep their splits.)
+  if (wide_tiles) {
+    auto partial_bytes = [&] {
+      int64_t n = 0;
+      for (int r = 0; r < num_reqs; ++r) {
+        const int64_t c = int64_t(query_start_loc[r + 1]) - query_start_loc[r];
+        const RequestSplit rs = request_split(c, context_lens[r]);
+        if (c > 0 && rs.pstride > 1) n += c * n_q_heads * rs.pstride;
+      }
+      return workspace_layout(n, head_dim).total;
+    };
+    while (tile_part < tile_split_cap && partial_bytes() > EDGERAG_ATTN_SCRATCH_BYTES)
+      tile_part = std::min(tile_split_cap, 2 * tile_part);
+  }
 
   // Scratch reused across calls on a thread: the planner runs once per step on the host.
   thread_local std::vector<PlanGroup> rows, tiles;
@@ -1136,12 +1173,10 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
     const int L = context_lens[r];
     int32_t* rq = reqs.data() + size_t(r) * kReqWords;
     const bool row = c * n_rep <= kMaxRowVecs;
-    // Workgroup-split rows: one item per part of the context (the waves split the part).
-    const int64_t slen = row ? (wg_rows ? wg_split_len(L) : split_len) : tile_split_len(L);
-    const int nsplit = c == 0 ? 0 : int((L + slen - 1) / slen);
-    // Slotted row requests write partials (and get merge rows) even when not split.
+    const RequestSplit rs = request_split(c, L);
+    const int64_t slen = rs.len;
+    const int nsplit = rs.n, pstride = rs.pstride;
     const bool slotted = slots > 0 && row;
-    const int pstride = slotted ? slots : nsplit;
     rq[R_NSPLIT] = nsplit;
     rq[R_SPLITLEN] = int32_t(slen);
     rq[R_PARTOFF] = int32_t(n_partials);

@@ -79,7 +79,7 @@ struct AttnLaunch {
   const int32_t* slots;
 };
 
-// Prefill tiles on MFMA (attention_prefill.hip): fp16, head_dim 64.
+// Prefill tiles on MFMA (attention_prefill.hip): fp16 and bf16, head_dim 64 and 128.
 #ifndef EDGERAG_TILE_ROWS
 #define EDGERAG_TILE_ROWS 128
 #endif
@@ -87,8 +87,11 @@ struct AttnLaunch {
 constexpr int kMfmaTileRows = EDGERAG_TILE_ROWS;
 constexpr int kMaxTileBlocks = 512;  // block ids one tile item stages in LDS (caps its split)
 // shared: one workgroup per CU (the rest of each CU is left to concurrently running rows).
-void launch_prefill_tiles_f16_d64(const AttnLaunch& a, int item_base, int count, bool shared);
-// Whether a pool of this size can use the MFMA tile kernel (buffer-resource addressing).
-bool prefill_tiles_supported(int32_t num_blocks, int32_t block_size);
+void launch_prefill_tiles(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int item_base,
+                          int count, bool shared);
+// Whether the MFMA tile kernel is built for this element type and head_dim.
+bool prefill_tile_shape(int32_t dtype, int32_t head_dim);
+// Whether a pool of this size can use it (buffer-resource addressing).
+bool prefill_tiles_supported(int32_t num_blocks, int32_t block_size, int32_t head_dim);
 
 }  // namespace edgerag

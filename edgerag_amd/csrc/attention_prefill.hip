@@ -1,28 +1,40 @@
-// Chunked-prefill attention tiles on CDNA4 matrix cores (fp16, head_dim 64).
+// Chunked-prefill attention tiles on CDNA4 matrix cores (fp16 and bf16, head_dim 64 and 128).
 //
 // A work item is (request, kv head, query tile of up to kMfmaTileRows virtual rows, KV split).
 // Virtual row rho is query token qb + rho / n_rep of query head h * n_rep + rho % n_rep, so all
 // heads of a GQA group share every K/V tile. Each wave owns 32 rows.
 //
 // Per 64-key tile:
-//   * the workgroup stages K row-major and V transposed (V^T[dim][key]) into one of two LDS
-//     buffers straight from the paged pool with raw buffer loads: keys without a valid block get
-//     an out-of-range offset and load zeros, no branch. A tile's loads are issued two tiles
-//     before it is staged, so HBM/L2 latency overlaps two tiles of matrix work; one barrier per
-//     tile. LDS rows are 128 bytes with the 16-byte chunk index XOR-swizzled by the row, so the
-//     MFMA operand reads and the staging writes are bank-conflict free.
-//   * each wave computes S^T = K Q^T with v_mfma_f32_32x32x16_f16: A = 32 keys x 16 dims from
-//     LDS, B = Q^T from registers (loaded once per item): per lane, 16 keys of one query.
-//   * online softmax in the log2 domain: Q is scaled by softmax_scale * log2(e) once per item
-//     (rounded to fp16, as torch's SDPA scales q before the product), and the S accumulators start
-//     at -m, so the MFMA leaves s - m and every probability is one v_exp_f32 with no FMA. The max
-//     m is only raised when a score beats it by 2^8 (lazy rescale; p <= 256 stays exact in fp16).
-//     Masks (causal k <= L - c + i, split end, invalid blocks) are applied only on tiles that need
-//     them.
-//   * O^T += V^T P^T with the same MFMA: the probabilities, packed to fp16, are already in the
-//     B-operand layout once the contraction index is permuted; V^T is stored in that permuted key
-//     order, so each A operand is one 16-byte LDS read. l accumulates the same fp16 p (v_dot2).
-// The output is O / l (fp16) or, for split items, fp32 partials merged by attn_combine_kernel.
+//   * K and V rows go from the paged pool straight into LDS (buffer_load ... lds, 16 bytes a lane):
+//     no staging registers and no LDS write instructions. A lane chooses which 16-byte chunk of
+//     its row it fetches, so the rows land XOR-swizzled and the operand reads are free of bank
+//     conflicts. Keys without a valid block get an out-of-range offset and zeros land. Two buffers
+//     of each: K of tile i + 2 and V of tile i + 1 are in flight while tile i is computed, with one
+//     barrier per tile.
+//   * S^T = K Q^T with v_mfma_f32_32x32x16: A = 32 keys x 16 dims from LDS, B = Q^T from registers
+//     (loaded once per item): per lane, 16 keys of one query.
+//   * online softmax in the log2 domain, p = exp2(s * scale * log2(e) - m). The max m is only
+//     raised when a score beats it by 2^8 (lazy rescale). Masks (causal k <= L - c + i, split end,
+//     invalid blocks) are applied only on tiles that need them.
+//   * O^T += V^T P^T with the same MFMA: the probabilities are already in the B-operand layout
+//     once the contraction index is permuted; the A operand is V read transposed out of its
+//     row-major LDS tile (ds_read_b64_tr_b16), four keys of one dim a lane and read.
+//   * fp16 at head_dim 64 rounds p to fp16 (l sums the same rounded p). The other shapes hold p
+//     in 32 bits: p = hi + lo with both halves in the 16-bit type, two MFMAs per step (the
+//     error of hi + lo is 2^-18 of p in bf16, 2^-22 in fp16, against 2^-9 and 2^-11 for the output
+//     rounding), and l sums the fp32 p.
+// A wave computes the scores of tile i + 1 while it exponentiates those of tile i, and scales and
+// reduces them while it accumulates P V of tile i: matrix and VALU work that do not depend on each
+// other alternate in the instruction stream. What bounds a tile now is instruction issue: at two
+// waves per SIMD a wave's 64-key tile takes ~1,600 cycles at head_dim 64 (130 VALU instructions of
+// ~4 cycles, 32 of them exponentials, and 16 MFMAs of 32 cycles) and ~3,000 at 128 (48 MFMAs);
+// taking out the loads, the exponentials or the P V products each gains about 10%.
+// Measured: bf16, 32/8 heads of 128, two 512-token slices at 2,048 and 4,096 keys beside 7 decodes
+// 4,388 us on the row kernel -> 123 us; four such slices at 4,096 keys, 129 GFLOP, 195 us (660
+// TFLOP/s). fp16 head_dim 64 against staging through registers with a transposing LDS write:
+// three slices beside 24 decodes 208 -> 206 us, a decoder's prefill iteration (4 layers)
+// 880 -> 864 us.
+// The output is O / l or, for split items, fp32 partials merged by attn_combine_kernel.
 #include "attention_plan.h"
 
 namespace edgerag {
@@ -30,17 +42,18 @@ namespace {
 
 using namespace plan;
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef float f2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kD = 64;
 #ifndef EDGERAG_ATTN_SHARED_PAD_KB
 #define EDGERAG_ATTN_SHARED_PAD_KB 48  // dynamic LDS of a shared-mode tile workgroup
-#endif
-#ifndef EDGERAG_ATTN_SHARED_TILES_PER_CU
-#define EDGERAG_ATTN_SHARED_TILES_PER_CU 1  // tile workgroups per CU that the pad allows
 #endif
 #ifndef EDGERAG_TILE_PRIO
 // Issue priority (s_setprio) of the tile waves. Beside the decode rows (shared mode) the VALU-
@@ -51,33 +64,21 @@ constexpr int kD = 64;
 #endif
 constexpr unsigned kSharedLdsPad = EDGERAG_ATTN_SHARED_PAD_KB * 1024;
 constexpr int kKeys = 64;            // keys per LDS tile
-constexpr int kRow = 64;             // halves per LDS row (K: one key; V^T: one dim)
 constexpr float kRescaleLog2 = 8.f;  // lazy rescale: p may grow to 2^8 before the max moves
 constexpr int kWaves = kMfmaTileRows / 32;
 constexpr int kThreads = kWaves * kWave;
-constexpr int kKChunks = kKeys * kD * 2 / 16;  // 16-byte chunks of a K tile (512)
-constexpr int kKPerThread = kKChunks / kThreads;
-#ifndef EDGERAG_TILE_VKEYS
-// Consecutive keys of one dim chunk a thread stages into V^T (2 or 4). With 2, the 256 (key pair,
-// dim chunk) units of a V tile give every thread of a 4-wave workgroup one, so no wave carries
-// the whole transpose (with 4 half the threads staged V and the other half waited at the barrier).
-#define EDGERAG_TILE_VKEYS 2
-#endif
-constexpr int kVKeys = EDGERAG_TILE_VKEYS;
-static_assert(kVKeys == 2 || kVKeys == 4, "V^T staging units of 2 or 4 keys");
-constexpr int kVGroups = kKeys / kVKeys;             // key groups of a V tile
-constexpr int kVPairs = kVGroups * (kD / 8);         // (key group, dim chunk) units of a V tile
-constexpr int kVPerThread = (kVPairs + kThreads - 1) / kThreads;
-static_assert(kKChunks % kThreads == 0, "K staging split");
-constexpr unsigned kStaticLds = 2 * kKeys * kRow * 2 + 2 * kD * kRow * 2 + kMaxTileBlocks * 4;
-constexpr unsigned kSharedTiles = EDGERAG_ATTN_SHARED_TILES_PER_CU;
-static_assert((kSharedTiles + 1) * (kStaticLds + kSharedLdsPad) > 160 * 1024 &&
-                  kSharedTiles * (kStaticLds + kSharedLdsPad) <= 160 * 1024,
-              "shared mode: the pad must leave room for exactly kSharedTiles tile workgroups per CU");
 
-// Byte offset handed to buffer loads for keys with no valid block: beyond num_records, so the
-// load returns zeros without a branch (the launcher keeps a head's pool slice below it).
-constexpr uint32_t kOutOfRange = 0xFFFFFFF0u;
+// Byte offset handed to buffer loads for keys with no valid block: beyond num_records (with any
+// chunk offset added), so zeros land without a branch (the launcher keeps a head's pool slice
+// below it).
+constexpr uint32_t kOutOfRange = 0xFFFFF000u;
+
+constexpr unsigned tile_lds(int d) { return 4 * kKeys * d * 2 + kMaxTileBlocks * 4; }
+static_assert(tile_lds(64) + kSharedLdsPad <= 160 * 1024 &&
+                  2 * (tile_lds(64) + kSharedLdsPad) > 160 * 1024 &&
+                  tile_lds(128) + kSharedLdsPad <= 160 * 1024 &&
+                  2 * (tile_lds(128) + kSharedLdsPad) > 160 * 1024,
+              "shared mode: the pad must leave room for exactly one tile workgroup per CU");
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -95,136 +96,123 @@ __device__ __forceinline__ float halves_sum(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-__device__ __forceinline__ f32x16 mfma32(h8 a, h8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+// The 16-bit element type of a tile kernel: vectors, matrix product, packing of probabilities.
+template <typename T>
+struct Elem;
+template <>
+struct Elem<f16> {
+  typedef h8 v8;
+  typedef h4 v4;
+  static __device__ __forceinline__ f32x16 mfma(v8 a, v8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ v4 pack4(float a, float b, float c, float d) {
+    return v4{_Float16(a), _Float16(b), _Float16(c), _Float16(d)};
+  }
+  // p[0], p[1] as two 16-bit words (round towards zero) and what the rounding left of each.
+  static __device__ __forceinline__ uint32_t head(f2 p) {
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p[0], p[1]));
+  }
+  static __device__ __forceinline__ uint32_t rest(f2 p, uint32_t hi) {
+    const h2 h = __builtin_bit_cast(h2, hi);
+    return __builtin_bit_cast(
+        uint32_t, __builtin_amdgcn_cvt_pkrtz(__builtin_fmaf(-float(h[0]), 1.f, p[0]),
+                                             __builtin_fmaf(-float(h[1]), 1.f, p[1])));
+  }
+};
+template <>
+struct Elem<bf16> {
+  typedef b8 v8;
+  typedef b4 v4;
+  static __device__ __forceinline__ f32x16 mfma(v8 a, v8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ v4 pack4(float a, float b, float c, float d) {
+    return v4{__bf16(a), __bf16(b), __bf16(c), __bf16(d)};
+  }
+  static __device__ __forceinline__ uint32_t head(f2 p) {
+    return __builtin_bit_cast(uint32_t, b2{__bf16(p[0]), __bf16(p[1])});
+  }
+  static __device__ __forceinline__ uint32_t rest(f2 p, uint32_t hi) {
+    return head(f2{p[0] - __uint_as_float(hi << 16), p[1] - __uint_as_float(hi & 0xFFFF0000u)});
+  }
+};
+
+// The LDS tile layouts. A row holds one key's D elements as D / 8 16-byte chunks; chunk c of key
+// k sits at slot c ^ swizzle(k). LDS serves 256 bytes (64 banks) a cycle, 16 slots: K operands are
+// read 16 bytes a lane down consecutive rows, so 16 consecutive rows (8 pairs of 128-byte rows,
+// or 16 of 256) must take different slots; V operands are read by ds_read_b64_tr_b16, where 32
+// lanes read 64 bytes (4 chunks) of each of 4 consecutive rows. (With only 8 slots told apart
+// the K reads of head_dim 64 and all reads of 128 took twice the LDS cycles.)
+template <int D>
+__device__ __forceinline__ int k_swizzle(int key) {
+  return D == 64 ? (key >> 1) & 7 : key & 15;
+}
+template <int D>
+__device__ __forceinline__ int v_swizzle(int key) {
+  return D == 64 ? (key & 3) << 1 : (key & 3) << 2;
 }
 
-__device__ __forceinline__ h8 buffer_load16(__amdgpu_buffer_rsrc_t rsrc, uint32_t byte_off) {
-  return __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, byte_off, 0, 0));
-}
-
-// Halves offset of 16-byte chunk `chunk` (0..7) of LDS row `row`, chunk index XOR-swizzled.
-__device__ __forceinline__ int lds_chunk(int row, int chunk) {
-  return row * kRow + ((chunk ^ (row & 7)) << 3);
-}
-
-// V^T keeps keys in the order the P.V k-steps consume them: within every 16 keys, bits 2 and 3
-// of the key index are swapped, so lane group g's keys {0-3, 8-11} + 4g of a k-step are one
-// contiguous 16-byte run.
-__device__ __forceinline__ int vt_slot(int key) {
-  return (key & ~12) | ((key & 4) << 1) | ((key & 8) >> 1);
-}
-
-struct StageRegs {
-  h8 k[kKPerThread];
-  h8 v[kVKeys * kVPerThread];
+template <bool B>
+struct Flag {
+  static constexpr bool value = B;
 };
 
 struct Geometry {
   int kb, ke, blk0, bs_shift, bs_mask;
 };
 
-// Block id of key position pos (-1 past the split or for an invalid table entry).
-__device__ __forceinline__ int block_of(const Geometry& geo, const int* __restrict__ sblk,
-                                        int pos) {
-  const int i = (pos >> geo.bs_shift) - geo.blk0;
-  return (pos < geo.ke && i < kMaxTileBlocks) ? sblk[i] : -1;
-}
-
-// Byte offset of (pos, 16-byte dim chunk dc) in one kv head's pool slice, or kOutOfRange.
-__device__ __forceinline__ uint32_t pool_offset(const Geometry& geo, int blk, int pos, int dc) {
-  return blk >= 0 ? ((uint32_t(blk) << geo.bs_shift) + uint32_t(pos & geo.bs_mask)) *
-                            uint32_t(kD * 2) + uint32_t(16 * dc)
-                  : kOutOfRange;
-}
-
-// The block ids one thread's staging loads of a 64-key tile need, looked up in LDS a tile before
-// the loads are issued (so issuing them waits on no LDS round trip).
-struct StageIds {
-  int k[kKPerThread];
-  int v[kVPerThread];
+// One kv head's slice of a pool.
+struct Slice {
+  const void* base;
+  uint32_t bytes;
 };
 
-// K: chunk c = tid + kThreads * j is key c / 8, dim chunk c % 8 (8 lanes fill one key row).
-// V: unit p = tid + kThreads * j is key group p % kVGroups (kVKeys keys), dim chunk p / kVGroups
-// (kVGroups lanes fill one V^T row).
-__device__ __forceinline__ void stage_ids(StageIds& ids, int tid, int k0, const Geometry& geo,
-                                          const int* __restrict__ sblk) {
+// 16 bytes a lane from byte offset `off` of the slice (zeros past its end) to dst + 16 lane in LDS.
+__device__ __forceinline__ void load_lds16(Slice s, char* dst, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(s.base), 0, s.bytes, 0x00020000),
+      (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
+}
+
+// One wave's share of a tile: load j fills the 64 / (D / 8) rows at dst + 1024 j lane by lane,
+// slot lane % (D / 8) of key lkey + 64 / (D / 8) j.
+template <int D, bool V, int N>
+__device__ __forceinline__ void fetch_tile(Slice s, char* dst, int lane, int lkey,
+                                           const uint32_t (&off)[N]) {
+  constexpr int kCh = D / 8;
 #pragma unroll
-  for (int j = 0; j < kKPerThread; ++j) ids.k[j] = block_of(geo, sblk, k0 + (tid + kThreads * j) / 8);
-#pragma unroll
-  for (int j = 0; j < kVPerThread; ++j) {
-    const int p = tid + kThreads * j;
-    ids.v[j] = (kVPairs % kThreads != 0 && p >= kVPairs)
-                   ? -1
-                   : block_of(geo, sblk, k0 + kVKeys * (p % kVGroups));
+  for (int j = 0; j < N; ++j) {
+    const int key = lkey + kWave / kCh * j;
+    const int chunk = (lane % kCh) ^ (V ? v_swizzle<D>(key) : k_swizzle<D>(key));
+    load_lds16(s, dst + j * 1024, __builtin_elementwise_add_sat(off[j], uint32_t(16 * chunk)));
   }
 }
 
-__device__ __forceinline__ void stage_load(StageRegs& st, const StageIds& ids, int tid, int k0,
-                                           const Geometry& geo, __amdgpu_buffer_rsrc_t krs,
-                                           __amdgpu_buffer_rsrc_t vrs) {
-#pragma unroll
-  for (int j = 0; j < kKPerThread; ++j) {
-    const int c = tid + kThreads * j;
-    st.k[j] = buffer_load16(krs, pool_offset(geo, ids.k[j], k0 + c / 8, c % 8));
-  }
-#pragma unroll
-  for (int j = 0; j < kVPerThread; ++j) {
-    const int p = tid + kThreads * j;
-    if (kVPairs % kThreads != 0 && p >= kVPairs) break;
-    const int a = p % kVGroups, b = p / kVGroups;
-    // The keys of a group share one block (blocks hold a multiple of 4 keys): one lookup, then
-    // consecutive rows; keys past the split still get the out-of-range offset.
-    const int pos = k0 + kVKeys * a;
-    const uint32_t base = pool_offset(geo, ids.v[j], pos, b);
-#pragma unroll
-    for (int kk = 0; kk < kVKeys; ++kk)
-      st.v[kVKeys * j + kk] = buffer_load16(
-          vrs, (base != kOutOfRange && pos + kk < geo.ke) ? base + uint32_t(kk * kD * 2)
-                                                          : kOutOfRange);
-  }
-}
-
-__device__ __forceinline__ void stage_store(const StageRegs& st, int tid,
-                                            _Float16* __restrict__ sk, _Float16* __restrict__ svt) {
-#pragma unroll
-  for (int j = 0; j < kKPerThread; ++j) {
-    const int c = tid + kThreads * j;
-    *reinterpret_cast<h8*>(sk + lds_chunk(c / 8, c % 8)) = st.k[j];
-  }
-#pragma unroll
-  for (int j = 0; j < kVPerThread; ++j) {
-    const int p = tid + kThreads * j;
-    if (kVPairs % kThreads != 0 && p >= kVPairs) break;
-    const int a = p % kVGroups, b = p / kVGroups;
-    const int slot = vt_slot(kVKeys * a);  // kVKeys-aligned: the group's keys stay contiguous
-#pragma unroll
-    for (int d = 0; d < 8; ++d) {
-      _Float16* dst = svt + lds_chunk(8 * b + d, slot >> 3) + (slot & 7);
-      if constexpr (kVKeys == 4) {
-        *reinterpret_cast<h4*>(dst) = h4{st.v[4 * j][d], st.v[4 * j + 1][d], st.v[4 * j + 2][d],
-                                         st.v[4 * j + 3][d]};
-      } else {
-        *reinterpret_cast<h2*>(dst) = h2{st.v[2 * j][d], st.v[2 * j + 1][d]};
-      }
-    }
-  }
-}
-
-// Two waves per SIMD: the register budget (256 per lane) keeps S, O and the staged tile in VGPRs.
+// Two waves per SIMD: the register budget (256 per lane) keeps two tiles' scores, O and Q in VGPRs.
+template <typename T, int D>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_prefill_mfma_kernel(
     const int32_t* __restrict__ plan, int32_t item_base, int32_t bs_shift,
     const int32_t* __restrict__ qsl, const int32_t* __restrict__ ctx,
     const int32_t* __restrict__ block_tables, int64_t bt_stride, int32_t num_blocks,
-    int32_t n_q_heads, const _Float16* __restrict__ q, int64_t q_st, int64_t q_sh,
-    const _Float16* __restrict__ kpool, const _Float16* __restrict__ vpool, int32_t n_kv_heads,
-    float scale_log2, _Float16* __restrict__ out,
+    int32_t n_q_heads, const T* __restrict__ q, int64_t q_st, int64_t q_sh,
+    const T* __restrict__ kpool, const T* __restrict__ vpool, int32_t n_kv_heads,
+    float scale_log2, T* __restrict__ out,
     int64_t o_st, int64_t o_sh, float2* __restrict__ part_ml, float* __restrict__ part_acc) {
-  __shared__ __align__(16) _Float16 sk[2][kKeys * kRow];
-  __shared__ __align__(16) _Float16 svt[2][kD * kRow];
-  __shared__ int sblk[kMaxTileBlocks];
+  using E = Elem<T>;
+  typedef typename E::v8 v8;
+  constexpr bool kSplit = !(__is_same(T, f16) && D == 64);  // p as hi + lo (see above)
+  constexpr int kCh = D / 8;                                 // 16-byte chunks of a row
+  constexpr int kKpi = kWave / kCh;                          // keys one wave load covers
+  constexpr int kLoads = kKeys / kKpi / kWaves;              // wave loads of a tile per wave
+  constexpr int kKs = D / 16;                                // 16-dim steps of S
+  constexpr int kDt = D / 32;                                // 32-dim tiles of O
+  // Separate arrays, not one with a buffer index: a load into one of them is then known not to
+  // alias reads of the others, so no read waits for the loads in flight.
+  __shared__ __align__(16) char sk0[kKeys * D * 2], sk1[kKeys * D * 2];
+  __shared__ __align__(16) char sv0[kKeys * D * 2], sv1[kKeys * D * 2];
+  __shared__ uint32_t sblk[kMaxTileBlocks];  // byte offset of each block in the head's slice
 
   if (EDGERAG_TILE_PRIO > 0) __builtin_amdgcn_s_setprio(EDGERAG_TILE_PRIO);
   const int32_t* it = plan + plan[H_ITEM_OFF] + int64_t(item_base + blockIdx.x) * kItemWords;
@@ -238,7 +226,8 @@ void attn_prefill_mfma_kernel(
   const int64_t head_base = int64_t(h) * num_blocks;
   const int block_size = 1 << bs_shift;
 
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int g = lane / 32, col = lane % 32;
   const int nrows = qc * n_rep;
   const int rho = wave * 32 + col;
@@ -266,7 +255,7 @@ void attn_prefill_mfma_kernel(
     for (int i = tid; i < nblk; i += kThreads) {
       const int32_t b = table[geo.blk0 + i];
       const bool ok = b >= 0 && b < num_blocks;
-      sblk[i] = ok ? b : -1;
+      sblk[i] = ok ? (uint32_t(b) << bs_shift) * uint32_t(D * 2) : kOutOfRange;
       any_bad |= ok ? 0 : 1;
     }
   }
@@ -276,59 +265,87 @@ void attn_prefill_mfma_kernel(
   // given. The scale (times log2 e) multiplies the fp32 dot products afterwards, like the decode
   // rows: scaling q first would round every q * scale to fp16, a score error that grows with the
   // score (scores of tens of nats, as with attention sinks, moved outputs by 3e-2).
-  h8 qop[4];
+  v8 qop[kKs];
   {
-    const _Float16* qp = q + int64_t(t) * q_st + int64_t(hq) * q_sh;
+    const T* qp = q + int64_t(t) * q_st + int64_t(hq) * q_sh;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      qop[ks] = active ? *reinterpret_cast<const h8*>(qp + 16 * ks + 8 * g) : h8{};
+    for (int ks = 0; ks < kKs; ++ks)
+      qop[ks] = active ? *reinterpret_cast<const v8*>(qp + 16 * ks + 8 * g) : v8{};
   }
-  f32x16 o0 = {}, o1 = {};  // O^T dims 0-31 and 32-63 of this lane's query
-  float m = -INFINITY;      // reference max of the log2-domain scores
-  float l = 0.f;
-  float nm = 0.f;           // -m (0 while m is -inf)
-  const f32x16 zero16 = {};
-  const h2 ones = {_Float16(1.f), _Float16(1.f)};
-
-  const uint32_t head_bytes = uint32_t(int64_t(num_blocks) * block_size * kD * 2);
-  const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<_Float16*>(kpool + head_base * block_size * kD), 0, head_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<_Float16*>(vpool + head_base * block_size * kD), 0, head_bytes, 0x00020000);
-
-  // One 64-key tile on staged LDS buffers (skb, svb).
-  auto tile = [&](int k0, const _Float16* skb, const _Float16* svb) {
-    // S^T = K Q^T: two 32-key tiles, 4 k-steps of 16 dims (dim chunk 2ks + g).
-    f32x16 s[2];
+  f32x16 o[kDt];  // O^T dims 32 dt + .. of this lane's query
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
+  for (int dt = 0; dt < kDt; ++dt) o[dt] = f32x16{};
+  float m = -INFINITY;  // reference max of the log2-domain scores
+  float l = 0.f;        // this lane half's keys only: the halves are added after the last tile
+  float nm = 0.f;       // -m (0 while m is -inf)
+
+  const uint32_t head_bytes = uint32_t(int64_t(num_blocks) * block_size * D * 2);
+  const Slice krs{kpool + head_base * block_size * D, head_bytes};
+  const Slice vrs{vpool + head_base * block_size * D, head_bytes};
+
+  // Staging: wave load j of wave w fills LDS rows kKpi (w kLoads + j) .. + kKpi - 1, lane by lane
+  // in order: key lkey + kKpi j of the tile, slot lane % kCh.
+  const int lkey = kKpi * kLoads * wave + lane / kCh, wave_lds = wave * kLoads * 1024;
+  // Row offsets of this thread's keys of the tile at k0 (a multiple of kKeys) in the head's pool
+  // slice: its block's, and the row in the block, which splits into a part of the thread and (for
+  // blocks of more than kKeys) a part of the tile. Sums past kOutOfRange saturate.
+  auto row_offsets = [&](int k0, uint32_t (&off)[kLoads]) {
+    const int i0 = (k0 >> bs_shift) - geo.blk0;
+    const uint32_t in_block = uint32_t(k0 & geo.bs_mask) * uint32_t(D * 2);
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        const h8 ka = *reinterpret_cast<const h8*>(skb + lds_chunk(32 * kt + col, 2 * ks + g));
-        s[kt] = mfma32(ka, qop[ks], ks == 0 ? zero16 : s[kt]);
-      }
+    for (int j = 0; j < kLoads; ++j) {
+      const int key = lkey + kKpi * j;
+      // Looked up in any case (the index clamped) and checked after: no branch around the read.
+      const uint32_t blk = sblk[min(i0 + (key >> bs_shift), kMaxTileBlocks - 1)];
+      const uint32_t row = uint32_t(key & geo.bs_mask) * uint32_t(D * 2) + in_block;
+      off[j] = key < ke - k0 ? __builtin_elementwise_add_sat(blk, row) : kOutOfRange;
     }
-    // log2-domain scores relative to the reference max: q.k * scale * log2(e) - m.
+  };
+
+  // S^T operand: keys 32 kt + col, dims 16 ks + 8 g .. + 7.
+  auto read_k = [&](const char* skb, int ks, int kt) {
+    const int key = 32 * kt + col;
+    return *reinterpret_cast<const v8*>(skb + key * (D * 2) +
+                                        16 * ((2 * ks + g) ^ k_swizzle<D>(key)));
+  };
+  // V^T operand of k-step st (keys 16 st + {0-3, 8-11} + 4 g) and dim tile dt: two transposing
+  // reads of 4 keys x 16 dims per 16 lanes.
+  auto read_v = [&](const char* svb, int st, int dt) {
+    union {
+      s4 half[2];
+      v8 all;
+    } u;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int key = 16 * st + 8 * i + 4 * g + (lane % 16) / 4;
+      const int dim = 32 * dt + 16 * ((lane / 16) % 2) + 4 * (lane % 4);
+      u.half[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (__attribute__((address_space(3))) s4*)(svb + key * (D * 2) +
+                                                  16 * ((dim / 8) ^ v_swizzle<D>(key)) +
+                                                  2 * (dim % 8)));
+    }
+    return u.all;
+  };
+
+  // Masks of the scores of the tile at k0 (already relative to m); their new maximum.
+  auto masked_max = [&](f32x16 (&s)[2], int k0, float tmax) {
+    const int key_end = min(ke - k0, kKeys);  // keys of this tile inside the split
+    if (k0 + kKeys - 1 <= wave_min_lim && key_end == kKeys && !item_has_bad) return tmax;
+    // Register i of tile kt holds key 32kt + (i%4) + 8(i/4) + 4g.
+    // Keys [0, vis_end + 4g) are visible: compared with constants, so that no key index of a
+    // lane is held in a register across the loop.
+    const int vis_end = min(key_end, lim - k0 + 1) - 4 * g;
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) s[kt][i] = __builtin_fmaf(s[kt][i], scale_log2, nm);
-    // Register i of tile kt holds key 32kt + (i%4) + 8(i/4) + 4g.
-    const int key_end = min(ke - k0, kKeys);  // keys of this tile inside the split
-    if (k0 + kKeys - 1 > wave_min_lim || key_end < kKeys) {
-      const int vis_end = min(key_end, lim - k0 + 1);  // keys [0, vis_end) are visible
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (32 * kt + (i & 3) + 8 * (i >> 2) + 4 * g >= vis_end) s[kt][i] = -INFINITY;
-    }
+      for (int i = 0; i < 16; ++i)
+        if (32 * kt + (i & 3) + 8 * (i >> 2) >= vis_end) s[kt][i] = -INFINITY;
     // Keys whose block id is invalid (never in a well-formed table): masked too.
     uint64_t bad = 0;
     if (item_has_bad) {
       const int bi =
           min(((k0 + min(lane, key_end - 1)) >> bs_shift) - geo.blk0, kMaxTileBlocks - 1);
-      bad = __ballot(lane < key_end && sblk[bi] < 0);
+      bad = __ballot(lane < key_end && sblk[bi] == kOutOfRange);
     }
     if (bad != 0) {
       // Lane group g's keys of tile kt are bits (i%4) + 8(i/4) of (bad_kt >> 4g).
@@ -340,14 +357,19 @@ void attn_prefill_mfma_kernel(
         if ((b1 >> bit) & 1u) s[1][i] = -INFINITY;
       }
     }
-    float tmax = s[0][0];
+    tmax = -INFINITY;
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, s[kt][i]);
+    return tmax;
+  };
+
+  // Lazy rescale before the tile whose scores (relative to m) are s with this lane half's
+  // maximum tmax: the reference max m only moves when a score beats it by 2^kRescaleLog2 (before
+  // the first visible score, m is -inf and s is absolute).
+  auto rescale = [&](f32x16 (&s)[2], float tmax) {
     tmax = halves_max(tmax);  // the other 16 keys of each 32-key tile
-    // Lazy rescale: the reference max m only moves when a score beats it by 2^kRescaleLog2 (the
-    // scores are s - m here; before the first visible score, m is -inf and s is absolute).
     const bool first = m == -INFINITY;
     const bool up = first ? tmax != -INFINITY : tmax > kRescaleLog2;
     if (__any(up)) {
@@ -356,117 +378,247 @@ void attn_prefill_mfma_kernel(
       if (up) m = first ? tmax : m + tmax;
       nm = m == -INFINITY ? 0.f : -m;
       l *= alpha;
-      o0 *= alpha;
-      o1 *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt) o[dt] *= alpha;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         s[0][i] -= shift;
         s[1][i] -= shift;
       }
     }
-
-    // P = exp2(s - m), packed to fp16 in the B-operand order of each k-step.
-    float lsum = 0.f;
-#pragma unroll
-    for (int st4 = 0; st4 < 4; ++st4) {
-      const int kt = st4 >> 1, half = st4 & 1;
-      h8 pb;
-#pragma unroll
-      for (int j = 0; j < 8; j += 2) {
-        const float p0 = exp2_fast(s[kt][8 * half + j]);
-        const float p1 = exp2_fast(s[kt][8 * half + j + 1]);
-        const h2 pp = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p0, p1));
-        pb[j] = pp[0];
-        pb[j + 1] = pp[1];
-        lsum = __builtin_amdgcn_fdot2(pp, ones, lsum, false);
-      }
-      const int vchunk = 4 * kt + 2 * half + g;  // permuted V^T slots of this k-step
-      o0 = mfma32(*reinterpret_cast<const h8*>(svb + lds_chunk(col, vchunk)), pb, o0);
-      o1 = mfma32(*reinterpret_cast<const h8*>(svb + lds_chunk(32 + col, vchunk)), pb, o1);
-    }
-    l += lsum;  // this half's keys only: the halves are added once, after the last tile
   };
 
-  // Register stages st0 / st1 alternate, so a tile's loads are issued two tiles before it is
-  // staged to LDS and have two tiles of matrix work to land. Loads past the split need no branch:
-  // their positions get out-of-range offsets and load zeros. One barrier per tile: it orders the
-  // tile's LDS writes before its reads, and every wave's reads of a buffer before its rewrite.
-  // The block ids of each stage's next loads are read from LDS one tile ahead (id0 / id1).
-  StageRegs st0, st1;
-  StageIds id0, id1;
-  stage_ids(id0, tid, kb, geo, sblk);
-  stage_ids(id1, tid, kb + kKeys, geo, sblk);
-  stage_load(st0, id0, tid, kb, geo, krs, vrs);
-  stage_load(st1, id1, tid, kb + kKeys, geo, krs, vrs);
-  stage_ids(id0, tid, kb + 2 * kKeys, geo, sblk);
-  stage_ids(id1, tid, kb + 3 * kKeys, geo, sblk);
-  for (int k0 = kb; k0 < ke; k0 += 2 * kKeys) {
-    stage_store(st0, tid, sk[0], svt[0]);
-    __syncthreads();
-    stage_load(st0, id0, tid, k0 + 2 * kKeys, geo, krs, vrs);
-    stage_ids(id0, tid, k0 + 4 * kKeys, geo, sblk);
-    if (wave_live) tile(k0, sk[0], svt[0]);
-    if (k0 + kKeys < ke) {
-      stage_store(st1, tid, sk[1], svt[1]);
-      __syncthreads();
-      stage_load(st1, id1, tid, k0 + 3 * kKeys, geo, krs, vrs);
-      stage_ids(id1, tid, k0 + 5 * kKeys, geo, sblk);
-      if (wave_live) tile(k0 + kKeys, sk[1], svt[1]);
+  // One tile: s holds its scores (masked, relative to m); with NEXT the scores of the tile at
+  // kn = k0 + kKeys are computed into sn on the way.
+  const f32x16 zero16 = {};
+  const h2 ones = {_Float16(1.f), _Float16(1.f)};
+  constexpr int kKAhead = 1, kAhead = 2;  // K steps / V operands read ahead of their MFMAs
+  auto tile = [&](auto next, const char* skb, const char* svb, f32x16 (&s)[2], f32x16 (&sn)[2],
+                  int kn) {
+    constexpr bool kNext = decltype(next)::value;
+    constexpr int kSteps = kNext ? kKs : 4;   // chunks of the first phase
+    constexpr int kPer = 32 / kSteps;         // probabilities exponentiated per chunk
+    uint32_t hi[16], lo[kSplit ? 16 : 1];     // P of k-step st: words 4 st .. 4 st + 3
+    float ls[2] = {0.f, 0.f};
+    v8 ka[kKAhead + 1][2];
+    if constexpr (kNext) {
+#pragma unroll
+      for (int c = 0; c < kKAhead; ++c) {
+        ka[c][0] = read_k(skb, c, 0);
+        ka[c][1] = read_k(skb, c, 1);
+      }
     }
+#pragma unroll
+    for (int c = 0; c < kSteps; ++c) {
+      if constexpr (kNext) {
+        if (c + kKAhead < kKs) {
+          ka[(c + kKAhead) % (kKAhead + 1)][0] = read_k(skb, c + kKAhead, 0);
+          ka[(c + kKAhead) % (kKAhead + 1)][1] = read_k(skb, c + kKAhead, 1);
+        }
+        sn[0] = E::mfma(ka[c % (kKAhead + 1)][0], qop[c], c == 0 ? zero16 : sn[0]);
+      }
+#pragma unroll
+      for (int w = c * kPer / 2; w < (c + 1) * kPer / 2; ++w) {
+        const int kt = w / 8, i = 2 * (w % 8);
+        const f2 p = {exp2_fast(s[kt][i]), exp2_fast(s[kt][i + 1])};
+        hi[w] = E::head(p);
+        if constexpr (kSplit) {
+          ls[0] += p[0];
+          ls[1] += p[1];
+          lo[w] = E::rest(p, hi[w]);
+        } else {
+          ls[w & 1] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, hi[w]), ones, ls[w & 1], false);
+        }
+        if constexpr (kNext)
+          if (w == c * kPer / 2 + kPer / 4) sn[1] = E::mfma(ka[c % (kKAhead + 1)][1], qop[c], c == 0 ? zero16 : sn[1]);
+      }
+    }
+    l += ls[0] + ls[1];
+    asm volatile("" : "+v"(l));  // summed here: sunk below, it would keep every p alive
+    // O^T += V^T P^T, and the next tile's scores scaled and reduced.
+    float tmax = -INFINITY;
+    v8 va[kAhead + 1];
+#pragma unroll
+    for (int n = 0; n < kAhead; ++n) va[n] = read_v(svb, n / kDt, n % kDt);
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+      union {
+        uint32_t w[4];
+        v8 v;
+      } ph, pl;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        ph.w[j] = hi[4 * st + j];
+        if constexpr (kSplit) pl.w[j] = lo[4 * st + j];
+      }
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt) {
+        const int n = st * kDt + dt;
+        if (n + kAhead < 4 * kDt)
+          va[(n + kAhead) % (kAhead + 1)] = read_v(svb, (n + kAhead) / kDt, (n + kAhead) % kDt);
+        o[dt] = E::mfma(va[n % (kAhead + 1)], ph.v, o[dt]);
+        if constexpr (kSplit) o[dt] = E::mfma(va[n % (kAhead + 1)], pl.v, o[dt]);
+        if constexpr (kNext) {
+          // log2-domain scores relative to the reference max: q.k * scale * log2(e) - m.
+#pragma unroll
+          for (int e = 8 / kDt * dt; e < 8 / kDt * (dt + 1); ++e) {
+            const int kt = st / 2, i = 8 * (st % 2) + e;
+            sn[kt][i] = __builtin_fmaf(sn[kt][i], scale_log2, nm);
+            tmax = fmaxf(tmax, sn[kt][i]);
+          }
+        }
+      }
+    }
+    if constexpr (kNext) rescale(sn, masked_max(sn, kn, tmax));
+  };
+  // The scores of the first tile alone.
+  auto first_scores = [&](const char* skb, f32x16 (&s)[2]) {
+#pragma unroll
+    for (int ks = 0; ks < kKs; ++ks)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+        s[kt] = E::mfma(read_k(skb, ks, kt), qop[ks], ks == 0 ? zero16 : s[kt]);
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        s[kt][i] = __builtin_fmaf(s[kt][i], scale_log2, nm);
+        tmax = fmaxf(tmax, s[kt][i]);
+      }
+    rescale(s, masked_max(s, kb, tmax));
+  };
+
+  // This wave's loads have landed; after the barrier, every wave's have, and every wave is done
+  // with the buffers of the tile before.
+  auto landed = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+  // Even tiles use buffers 0 and offsets off0, odd tiles buffers 1 and off1. While tile i is
+  // computed, K of tile i + 2 and V of tile i + 1 are on their way (tiles past the split load
+  // zeros).
+  uint32_t off0[kLoads], off1[kLoads];
+  auto advance_even = [&](int k0) {
+    landed();
+    fetch_tile<D, false>(krs, sk0 + wave_lds, lane, lkey, off0);
+    fetch_tile<D, true>(vrs, sv1 + wave_lds, lane, lkey, off1);
+    row_offsets(k0 + 3 * kKeys, off1);
+  };
+  auto advance_odd = [&](int k0) {
+    landed();
+    fetch_tile<D, false>(krs, sk1 + wave_lds, lane, lkey, off1);
+    fetch_tile<D, true>(vrs, sv0 + wave_lds, lane, lkey, off0);
+    row_offsets(k0 + 3 * kKeys, off0);
+  };
+  row_offsets(kb, off0);
+  fetch_tile<D, false>(krs, sk0 + wave_lds, lane, lkey, off0);
+  row_offsets(kb + kKeys, off1);
+  landed();
+  fetch_tile<D, false>(krs, sk1 + wave_lds, lane, lkey, off1);
+  fetch_tile<D, true>(vrs, sv0 + wave_lds, lane, lkey, off0);
+  row_offsets(kb + 2 * kKeys, off0);
+  const int last = kb + (ke - kb - 1) / kKeys * kKeys;  // first key of the last tile
+  if (!wave_live) {  // this wave only stages
+    for (int k0 = kb; k0 <= last; k0 += 2 * kKeys) {
+      advance_even(k0);
+      if (k0 < last) advance_odd(k0 + kKeys);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return;
   }
+  f32x16 s0[2], s1[2];
+  first_scores(sk0, s0);
+  int k0 = kb;
+  const char* svl = sv0;  // V of the last tile
+  for (; k0 < last; k0 += 2 * kKeys) {
+    advance_even(k0);
+    tile(Flag<true>{}, sk1, sv0, s0, s1, k0 + kKeys);
+    if (k0 + kKeys >= last) {
+      s0[0] = s1[0];
+      s0[1] = s1[1];
+      svl = sv1;
+      break;
+    }
+    advance_odd(k0 + kKeys);
+    tile(Flag<true>{}, sk0, sv1, s1, s0, k0 + 2 * kKeys);
+  }
+  landed();
+  tile(Flag<false>{}, sk0, svl, s0, s1, 0);
+  // No load may still be on its way into this workgroup's LDS when the workgroup ends.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   l = halves_sum(l);
 
   if (!active) return;
   // O^T register i of dim tile dt holds dim 32dt + (i%4) + 8(i/4) + 4g of this lane's query.
   if (nsplit == 1) {
     const float inv = 1.f / fmaxf(l, 1.17549435e-38f);
-    _Float16* op = out + int64_t(t) * o_st + int64_t(hq) * o_sh;
+    T* op = out + int64_t(t) * o_st + int64_t(hq) * o_sh;
+    const bool vec_out =
+        (reinterpret_cast<uintptr_t>(out) & 7) == 0 && o_st % 4 == 0 && o_sh % 4 == 0;
 #pragma unroll
-    for (int qd = 0; qd < 4; ++qd) {
-      const int d0 = 8 * qd + 4 * g;
-      *reinterpret_cast<h4*>(op + d0) =
-          h4{_Float16(o0[4 * qd] * inv), _Float16(o0[4 * qd + 1] * inv),
-             _Float16(o0[4 * qd + 2] * inv), _Float16(o0[4 * qd + 3] * inv)};
-      *reinterpret_cast<h4*>(op + 32 + d0) =
-          h4{_Float16(o1[4 * qd] * inv), _Float16(o1[4 * qd + 1] * inv),
-             _Float16(o1[4 * qd + 2] * inv), _Float16(o1[4 * qd + 3] * inv)};
-    }
+    for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) {
+        T* dst = op + 32 * dt + 8 * qd + 4 * g;
+        const typename E::v4 v = E::pack4(o[dt][4 * qd] * inv, o[dt][4 * qd + 1] * inv,
+                                          o[dt][4 * qd + 2] * inv, o[dt][4 * qd + 3] * inv);
+        if (vec_out) {
+          *reinterpret_cast<typename E::v4*>(dst) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dst[e] = __builtin_bit_cast(T, v[e]);
+        }
+      }
   } else {
     // Partials carry the max in the log2 domain, like the decode kernels'.
     const int64_t idx = int64_t(part_off) + (int64_t(t - q0) * n_q_heads + hq) * pstride + split;
     if (g == 0) part_ml[idx] = make_float2(m, l);
-    float* pa = part_acc + idx * kD;
+    float* pa = part_acc + idx * D;
 #pragma unroll
-    for (int qd = 0; qd < 4; ++qd) {
-      const int d0 = 8 * qd + 4 * g;
-      *reinterpret_cast<float4*>(pa + d0) =
-          make_float4(o0[4 * qd], o0[4 * qd + 1], o0[4 * qd + 2], o0[4 * qd + 3]);
-      *reinterpret_cast<float4*>(pa + 32 + d0) =
-          make_float4(o1[4 * qd], o1[4 * qd + 1], o1[4 * qd + 2], o1[4 * qd + 3]);
-    }
+    for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd)
+        *reinterpret_cast<float4*>(pa + 32 * dt + 8 * qd + 4 * g) =
+            make_float4(o[dt][4 * qd], o[dt][4 * qd + 1], o[dt][4 * qd + 2], o[dt][4 * qd + 3]);
   }
 }
 
+template <typename T, int D>
+void launch_tiles(const AttnLaunch& a, int item_base, int count, bool shared) {
+  // Shared mode reserves unused dynamic LDS so that a second workgroup no longer fits a CU's
+  // 160 KiB (the static arrays take 34 or 66 KiB): the tiles then hold one of each SIMD's two
+  // register halves and decode waves keep the other.
+  const unsigned pad = shared ? kSharedLdsPad : 0;
+  hipLaunchKernelGGL((attn_prefill_mfma_kernel<T, D>), dim3(count), dim3(kThreads), pad, a.s,
+                     a.plan, item_base, log2_exact(a.bs), a.qsl, a.ctx, a.bt, a.bt_stride, a.nb,
+                     a.hq, static_cast<const T*>(a.q), a.q_st, a.q_sh,
+                     static_cast<const T*>(a.kp), static_cast<const T*>(a.vp), a.hkv,
+                     a.scale_log2, static_cast<T*>(a.out), a.o_st, a.o_sh, a.ml, a.pacc);
+}
 }  // namespace
 
-bool prefill_tiles_supported(int32_t num_blocks, int32_t block_size) {
-  // Power-of-two blocks of at least 4 keys (shift addressing; a V key quad never straddles a
-  // block), and one kv head's slice of a pool must fit a buffer resource, below kOutOfRange.
-  return log2_exact(block_size) >= 2 &&
-         int64_t(num_blocks) * block_size * kD * 2 < int64_t(kOutOfRange);
+bool prefill_tile_shape(int32_t dtype, int32_t head_dim) {
+  return (dtype == EDGERAG_F16 || dtype == EDGERAG_BF16) && (head_dim == 64 || head_dim == 128);
 }
 
-void launch_prefill_tiles_f16_d64(const AttnLaunch& a, int item_base, int count, bool shared) {
-  // Shared mode reserves unused dynamic LDS so that a second workgroup no longer fits a CU's
-  // 160 KiB (the static arrays take ~34 KiB): the tiles then hold one of each SIMD's two register
-  // halves and decode waves keep the other.
-  const unsigned pad = shared ? kSharedLdsPad : 0;
-  hipLaunchKernelGGL(attn_prefill_mfma_kernel, dim3(count), dim3(kThreads), pad, a.s, a.plan,
-                     item_base, log2_exact(a.bs), a.qsl, a.ctx, a.bt, a.bt_stride, a.nb, a.hq,
-                     static_cast<const _Float16*>(a.q), a.q_st, a.q_sh,
-                     static_cast<const _Float16*>(a.kp), static_cast<const _Float16*>(a.vp),
-                     a.hkv, a.scale_log2, static_cast<_Float16*>(a.out), a.o_st,
-                     a.o_sh, a.ml, a.pacc);
+bool prefill_tiles_supported(int32_t num_blocks, int32_t block_size, int32_t head_dim) {
+  // Power-of-two blocks of at least 4 keys (shift addressing), and one kv head's slice of a pool
+  // must fit a buffer resource, below kOutOfRange.
+  return log2_exact(block_size) >= 2 &&
+         int64_t(num_blocks) * block_size * head_dim * 2 < int64_t(kOutOfRange);
+}
+
+void launch_prefill_tiles(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int item_base,
+                          int count, bool shared) {
+  const bool half = dtype == EDGERAG_F16;
+  if (head_dim == 64) {
+    if (half) launch_tiles<f16, 64>(a, item_base, count, shared);
+    else launch_tiles<bf16, 64>(a, item_base, count, shared);
+  } else {
+    if (half) launch_tiles<f16, 128>(a, item_base, count, shared);
+    else launch_tiles<bf16, 128>(a, item_base, count, shared);
+  }
 }
 
 }  // namespace edgerag

@@ -439,6 +439,20 @@ def _mixed(slices, decodes):
     return np.concatenate([[0], np.cumsum(q)]).astype(np.int32), np.array(ctx, np.int32)
 
 
+@pytest.mark.parametrize("n_q,n_kv", [(32, 32), (32, 8), (9, 3)])
+def test_wide_tile_partials_fit_the_static_scratch(n_q, n_kv) -> None:
+    """The partials of bf16 and head_dim-128 tiles fit the no-alloc entry's scratch for every
+    slice that one request of 8,192 positions can send (a split plan's items, 66 KB each, would
+    pass it where the tiles just miss one per CU), and splits stay whole 64-key tiles."""
+    for c in (9, 100, 500, 512, 1020, 1024, 2040):
+        for n in (1, 2, 3):
+            qsl, ctx = _mixed([(c, 4000)] * n, [5000])
+            plan, nbytes = kernels.make_plan_host(qsl, ctx, n_q, n_kv, 128, 16, 512, torch.bfloat16)
+            assert nbytes <= _lib.ATTN_SCRATCH_BYTES
+            _items, reqs = decode_plan(plan)
+            assert all(int(reqs[r][1]) % 64 == 0 for r in range(n))
+
+
 @pytest.mark.parametrize("slices,decodes,force,overlap", [
     # config 3: 384 tiles (every CU at one workgroup) beside 24 decodes reading 707 MB
     ([(512, 0), (512, 3584), (512, 6656)], "cfg3", False, 1),

@@ -393,6 +393,33 @@ def test_fp16_prefill_chunk_edges(device, c, past) -> None:
     torch.testing.assert_close(got.float(), expected, **FP16_TOL)
 
 
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 128),
+                                     (torch.bfloat16, 128)])
+@pytest.mark.parametrize("n_q,n_kv", [(4, 4), (6, 2), (8, 2)])
+def test_wide_prefill_tile_edges(device, dtype, d, n_q, n_kv) -> None:
+    """The tiles that hold p in 32 bits: one token past the row limit, one short of and past a
+    128-row tile, chunks below, at and past a 64-key tile, odd prefixes and a split context, all
+    in one batch whose unwritten pool rows are NaN, against the float64 softmax. The error is the
+    rounding of the output (2^-9 relative for bf16, 2^-11 for fp16) plus that of hi + lo
+    (2^-17, 2^-22)."""
+    rep = n_q // n_kv
+    chunks = [8 // rep + 1, 64, 65, 128 // rep - 1, 128 // rep + 1, 200]
+    lens = [c + p for c, p in zip(chunks, [0, 0, 13, 64, 250, 1900])]
+    kp, vp, tables, qsl, q, bt = _ragged_case(lens, chunks, n_q, n_kv, d, dtype, 7 * d + n_q)
+    for r, L in enumerate(lens):  # rows past a context's end, in its last block
+        if L % BLOCK_SIZE:
+            kp[:, tables[r][-1], L % BLOCK_SIZE:] = float("nan")
+            vp[:, tables[r][-1], L % BLOCK_SIZE:] = float("nan")
+    got = _run_ragged(device, kp, vp, qsl, lens, bt, q, d**-0.5).double()
+    u = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-11
+    for r, (L, c) in enumerate(zip(lens, chunks)):
+        for h in (0, n_q - 1):
+            k = op.gather_pool(kp.float(), tables[r], L)[h // rep]
+            v = op.gather_pool(vp.float(), tables[r], L)[h // rep]
+            ref = oa.attention_f64(q[qsl[r] : qsl[r + 1], h].float(), k, v, L - c, d**-0.5)
+            torch.testing.assert_close(got[qsl[r] : qsl[r + 1], h], ref, rtol=2 * u, atol=u / 64)
+
+
 def test_cfg2_shape_decode_batch_fp16(device) -> None:
     """BASELINE config 2 at full shape: 32 decodes, L ~ U[256, 7472], 32/32 heads, d 64,
     16,384-block pool (1 GiB per pool), seeded-shuffled tables."""
