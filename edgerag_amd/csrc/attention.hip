@@ -138,6 +138,10 @@ constexpr int kMaxSplitBlocks = 64;  // one block id per lane in the decode kern
 #endif
 constexpr int kMinTileSplit = EDGERAG_MIN_TILE_SPLIT;  // keys: tiles split no finer than this
 constexpr int kTargetTiles = EDGERAG_TARGET_TILES;  // prefill tile items a batch aims for
+// 16-row fp32 tiles up to which a batch takes them, at head_dim 64 and 128; past that, 32 rows.
+// 32 against 16 rows (us): head_dim 64, 360 tiles 18.1 / 14.3, 1,200 39.7 / 31.0, 2,048 long ones
+// 244 / 258; head_dim 128, 320 tiles 25.5 / 23.6, 960 49.6 / 58.0, 2,048 475 / 552.
+constexpr int kF32Tiles16D64 = 1536, kF32Tiles16D128 = 512;
 constexpr int kPlanCUs = 256;  // compute units the planner fills (MI355X)
 // K/V bytes decode rows must read for the planner to put them beside prefill tiles.
 constexpr int64_t kOverlapRowBytes = int64_t(256) << 20;
@@ -897,8 +901,8 @@ void dispatch_rows_qr(const Launch& a, int qr, int base, int count, int limit_wo
   }
 }
 
-// Tile items (prefill slices) first: the MFMA tile kernel for fp16 and bf16 with head_dim 64 or
-// 128, the general row kernel with 8 query vectors per pass otherwise. Row items: the fast decode kernel when
+// Tile items (prefill slices) first: an MFMA tile kernel for head_dim 64 or 128, the general row
+// kernel with 8 query vectors per pass otherwise. Row items: the fast decode kernel when
 // every split's load groups stay inside one block, the general kernel otherwise.
 template <typename T, int D>
 int run_items(const Launch& a, const int32_t* ph, int parts) {
@@ -912,6 +916,11 @@ int run_items(const Launch& a, const int32_t* ph, int parts) {
       } else {
         dispatch_rows_qr<T, D>(a, 8, n_row, n_items - n_row, H_N_ITEMS);
       }
+    } else if constexpr (D == 64 || D == 128) {
+      if (ph[H_TILE_KIND] >= 2 && prefill_f32_supported(a.nb, a.bs, D))
+        launch_prefill_f32(a, D, ph[H_TILE_KIND] == 2 ? 16 : 32, n_row, n_items - n_row);
+      else
+        dispatch_rows_qr<T, D>(a, 8, n_row, n_items - n_row, H_N_ITEMS);
     } else {
       dispatch_rows_qr<T, D>(a, 8, n_row, n_items - n_row, H_N_ITEMS);
     }
@@ -974,8 +983,21 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
   const int n_rep = n_q_heads / n_kv_heads;
   // Prefill tiles on MFMA: 128 virtual rows (token x head-in-group).
   const bool mfma_tiles = prefill_tile_shape(dtype, head_dim) && n_rep <= kMfmaTileRows;
-  const bool wide_tiles = mfma_tiles && !(dtype == EDGERAG_F16 && head_dim == 64);
-  const int tile_rows = mfma_tiles ? kMfmaTileRows / n_rep : kQTile;
+  // In fp32 on 16 or 32 virtual rows: 16 for batches of few tiles (short prompts, where the chain
+  // of one workgroup's chunks is the time), else 32, which read K and V half as often.
+  int tile_kind = mfma_tiles ? 1 : 0;
+  int tile_rows = mfma_tiles ? kMfmaTileRows / n_rep : kQTile;
+  if (dtype == EDGERAG_F32 && n_rep <= 16 && prefill_f32_supported(1, block_size, head_dim)) {
+    int64_t tiles16 = 0;
+    for (int r = 0; r < num_reqs; ++r) {
+      const int64_t c = int64_t(query_start_loc[r + 1]) - query_start_loc[r];
+      if (c * n_rep > kMaxRowVecs) tiles16 += (c * n_rep + 15) / 16 * n_kv_heads;
+    }
+    tile_kind = tiles16 <= (head_dim == 64 ? kF32Tiles16D64 : kF32Tiles16D128) ? 2 : 3;
+    tile_rows = (tile_kind == 2 ? 16 : 32) / n_rep;
+  }
+  const bool wide_tiles =
+      tile_kind > 1 || (mfma_tiles && !(dtype == EDGERAG_F16 && head_dim == 64));
   int64_t work = 0;       // KV token-heads the decode rows read, to size their splits
   int64_t tile_work = 0;  // tile x keys of the prefill slices, to size theirs
   int64_t n_tiles = 0;    // prefill tile items before any KV split
@@ -1246,7 +1268,7 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
   plan[H_MAX_SPLIT_BLOCKS] = wg_rows ? wg_split_blocks : split_blocks;
   plan[H_N_COMBINE] = int32_t(combine.size() / kCombineWords);
   plan[H_COMBINE_OFF] = int32_t(combine_off);
-  plan[H_TILE_KIND] = mfma_tiles ? 1 : 0;
+  plan[H_TILE_KIND] = tile_kind;
   plan[H_ROW_WAVES] = row_waves;
   plan[H_OVERLAP] = overlap ? 1 : 0;
   plan[H_SLOTS] = slots;

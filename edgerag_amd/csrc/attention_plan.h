@@ -33,7 +33,8 @@ enum Header {
   H_MAX_SPLIT_BLOCKS,  // blocks in the longest decode split
   H_N_COMBINE,         // rows (query tokens of split requests) attn_combine_kernel merges
   H_COMBINE_OFF,       // word offset of the combine list
-  H_TILE_KIND,         // 0: prefill tiles run on the row kernel, 1: on the MFMA tile kernel
+  H_TILE_KIND,         // 0: prefill tiles run on the row kernel, 1: on the MFMA tile kernel,
+                       // 2 / 3: on the fp32 MFMA tile kernel with 16 / 32 rows
   H_ROW_WAVES,         // 0: decode rows split across workgroups (partials + combine list);
                        // W > 0: one workgroup per row item, its W waves split the keys and
                        // merge in LDS (partials only where a context is cut into parts)
@@ -93,5 +94,9 @@ void launch_prefill_tiles(const AttnLaunch& a, int32_t dtype, int32_t head_dim, 
 bool prefill_tile_shape(int32_t dtype, int32_t head_dim);
 // Whether a pool of this size can use it (buffer-resource addressing).
 bool prefill_tiles_supported(int32_t num_blocks, int32_t block_size, int32_t head_dim);
+
+// Prefill tiles in fp32 (attention_prefill_f32.hip), head_dim 64 and 128: 16 or 32 virtual rows.
+void launch_prefill_f32(const AttnLaunch& a, int32_t head_dim, int rows, int item_base, int count);
+bool prefill_f32_supported(int32_t num_blocks, int32_t block_size, int32_t head_dim);
 
 }  // namespace edgerag

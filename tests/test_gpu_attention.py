@@ -394,10 +394,11 @@ def test_fp16_prefill_chunk_edges(device, c, past) -> None:
 
 
 @pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 128),
-                                     (torch.bfloat16, 128)])
+                                     (torch.bfloat16, 128), (torch.float32, 64),
+                                     (torch.float32, 128)])
 @pytest.mark.parametrize("n_q,n_kv", [(4, 4), (6, 2), (8, 2)])
 def test_wide_prefill_tile_edges(device, dtype, d, n_q, n_kv) -> None:
-    """The tiles that hold p in 32 bits: one token past the row limit, one short of and past a
+    """The tiles that hold p in 32 bits (the fp32 ones too): one token past the row limit, one short of and past a
     128-row tile, chunks below, at and past a 64-key tile, odd prefixes and a split context, all
     in one batch whose unwritten pool rows are NaN, against the float64 softmax. The error is the
     rounding of the output (2^-9 relative for bf16, 2^-11 for fp16) plus that of hi + lo
@@ -411,13 +412,38 @@ def test_wide_prefill_tile_edges(device, dtype, d, n_q, n_kv) -> None:
             kp[:, tables[r][-1], L % BLOCK_SIZE:] = float("nan")
             vp[:, tables[r][-1], L % BLOCK_SIZE:] = float("nan")
     got = _run_ragged(device, kp, vp, qsl, lens, bt, q, d**-0.5).double()
-    u = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-11
+    u = {torch.bfloat16: 2.0**-9, torch.float16: 2.0**-11}.get(dtype)
+    tol = FP32_TOL if u is None else dict(rtol=2 * u, atol=u / 64)
     for r, (L, c) in enumerate(zip(lens, chunks)):
         for h in (0, n_q - 1):
             k = op.gather_pool(kp.float(), tables[r], L)[h // rep]
             v = op.gather_pool(vp.float(), tables[r], L)[h // rep]
             ref = oa.attention_f64(q[qsl[r] : qsl[r + 1], h].float(), k, v, L - c, d**-0.5)
-            torch.testing.assert_close(got[qsl[r] : qsl[r + 1], h], ref, rtol=2 * u, atol=u / 64)
+            torch.testing.assert_close(got[qsl[r] : qsl[r + 1], h], ref, **tol)
+
+
+@pytest.mark.parametrize("dtype,d,reqs", [(torch.float16, 128, 1), (torch.float32, 64, 1),
+                                          (torch.float32, 128, 12)])
+@pytest.mark.parametrize("bs", [1, 4, 32, 128])
+def test_wide_prefill_tiles_at_other_block_sizes(device, dtype, d, reqs, bs) -> None:
+    """Blocks smaller and larger than a 64-key tile (the row kernel takes blocks of less than 4 in
+    fp16), a bad block id in the table's tail, and enough requests for 32-row fp32 tiles."""
+    g = seeded(bs + d)
+    c, L, h = 70, 333, 2
+    nb = -(-L // bs)
+    kp, vp = (torch.randn(h, reqs * nb, bs, d, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(reqs * c, 2 * h, d, generator=g).to(dtype)
+    bt = torch.randperm(reqs * nb, generator=g).view(reqs, nb)
+    table = torch.cat([bt, torch.full((reqs, 1), -1)], 1).int().numpy()
+    got = ragged_paged_attention(
+        q.to(device), kp.to(device), vp.to(device), np.arange(reqs + 1, dtype=np.int32) * c,
+        np.full(reqs, L, np.int32), table, d**-0.5).cpu().double()
+    tol = FP32_TOL if dtype == torch.float32 else FP16_TOL
+    for r in range(reqs):
+        for hq in range(2 * h):
+            k, v = (p[hq // 2, bt[r]].reshape(-1, d)[:L].float() for p in (kp, vp))
+            ref = oa.attention_f64(q[r * c : (r + 1) * c, hq].float(), k, v, L - c, d**-0.5)
+            torch.testing.assert_close(got[r * c : (r + 1) * c, hq], ref, **tol)
 
 
 def test_cfg2_shape_decode_batch_fp16(device) -> None:
