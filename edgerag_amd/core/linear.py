@@ -178,9 +178,16 @@ class QuantLinear(LinearBase):
         )
 
     def forward(self, x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+        # nn.Module finds a buffer by name after its own attributes fail (0.6 us each): one look
+        # into the dict that holds them, and the attributes only if they are not there.
+        buffers, config = self._buffers, self.config
+        try:
+            packed, scales, bias = buffers["packed"], buffers["scales"], buffers["bias"]
+        except KeyError:
+            packed, scales, bias = self.packed, self.scales, self.bias
         return kernels.quant_linear(
-            x, self.packed, self.scales, self.bias, self.in_features, self.out_features,
-            self.config.bits, self.config.group_size, out=out,
+            x, packed, scales, bias, self.in_features, self.out_features, config.bits,
+            config.group_size, out=out,
         )
 
     def rope_append(self, x: torch.Tensor, positions, cos, sin, n_q_heads: int, n_kv_heads: int,
