@@ -119,6 +119,13 @@ constexpr int32_t kPlanVersion = plan::kVersion;
 #endif
 constexpr int kRowWgWaves = EDGERAG_ROW_WG_WAVES;
 constexpr int kRowPartWaves = EDGERAG_ROW_PART_WAVES;
+// Rows of the GQA kernel at head_dim 128: workgroups of kGqaWaves = 4 waves, over a part of a context
+// or a whole one (then at most kGqaWaveTokens a wave). A wave's two V buffers take 16 KB of LDS,
+// so 8 waves fill a CU alone: parts of 4 against 8 waves, bf16 32/8 heads, 8 requests of 512-2,048
+// tokens 16.6 / 21.0 us; one of 2,048 9.6 / 11.0. Whole contexts in 4 waves of up to 512 tokens against
+// KV splits past 256 a wave, 32 requests of up to 1,500 tokens 27.1 / 25.5 us, but no merge launch to
+// capture. At head_dim 64 the buffers take half and rows keep the waves of the other kernel.
+constexpr int kGqaWaveTokens = 512;
 constexpr int kRowTargetWgs = EDGERAG_ROW_TARGET_WGS;
 constexpr int kRowMinWaveTokens = EDGERAG_ROW_MIN_WAVE_TOKENS;
 constexpr int kMaxRowVecs = 8;  // query vectors a decode item may carry (c * n_rep)
@@ -872,6 +879,16 @@ template <typename T, int D>
 void dispatch_decode_qr(const Launch& a, int qr, int base, int count, int limit_word,
                         int waves) {
   constexpr int U = D >= 256 ? 2 : kDecodeU;
+  // Two or more query vectors a row: the matrix cores (attention_decode_gqa.hip), where the VALU
+  // kernel is bound by its arithmetic (bf16 32/8 heads of 128, 48 requests 216 -> 159 us; two vectors,
+  // fp16 16/8 of 128, 32 requests, 77.6 -> 74.7).
+  if constexpr (!__is_same(T, float) && (D == 64 || D == 128)) {
+    constexpr int32_t kType = __is_same(T, f16) ? EDGERAG_F16 : EDGERAG_BF16;
+    if (decode_gqa_supported(a, kType, D, qr, waves)) {
+      launch_decode_gqa(a, kType, D, base, count, limit_word, waves);
+      return;
+    }
+  }
   // Workgroup rows (up to 16 waves, 128 registers per lane) take at most 4 query vectors per
   // pass: a pass of 8 spills 236-264 B per lane to scratch (fp16; ~430 B for bf16, whose query
   // vectors are fp32). GQA groups of 8 then take two passes over the keys, the second mostly from
@@ -1066,13 +1083,26 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
   const int64_t wave_cap = std::min<int64_t>(
       overlap && row_items >= kPlanCUs ? EDGERAG_ROW_WG_PART_TILES : EDGERAG_ROW_WG_PART,
       int64_t(kMaxSplitBlocks) * block_size);
-  const int64_t part_cap = int64_t(kRowWgWaves) * round_up(wave_cap, block_size);
+  // Rows of 2 to 8 query vectors run on the GQA kernel (attention_decode_gqa.hip).
+  int64_t max_vecs = 0;
+  for (int r = 0; r < num_reqs; ++r) {
+    const int64_t v = (int64_t(query_start_loc[r + 1]) - query_start_loc[r]) * n_rep;
+    if (v <= kMaxRowVecs) max_vecs = std::max(max_vecs, v);
+  }
+  const bool gqa_rows =
+      head_dim == 128 && decode_gqa_shape(dtype, head_dim, int(max_vecs), block_size);
+  const int full_waves = gqa_rows ? kGqaWaves : kRowWgWaves;
+  const int part_waves = gqa_rows ? kGqaWaves : kRowPartWaves;
+  const int64_t part_cap =
+      int64_t(full_waves) *
+      round_up(gqa_rows ? std::min<int64_t>(kGqaWaveTokens, kMaxSplitBlocks * block_size)
+                        : wave_cap, block_size);
   bool wg_rows = false;
   int row_waves = 0;
   int slots = 0;        // partial slots per (token, q head) of the row requests (0: nsplit)
   int64_t wg_part = 0;  // longest part of a context one row workgroup takes (0: whole contexts)
   if (wg_capable && kRowTargetWgs > 0 && row_items < kPlanCUs) {
-    // Parts take kRowPartWaves waves: single-sequence attention over 6,758 tokens measured
+    // Parts take kRowPartWaves (or kGqaWaves) waves: single-sequence attention over 6,758 tokens measured
     // 17.7 us at 8 waves against 21.5 us at 16 and 19.4 us at 4 (with the merge launch).
     // At most kRowTargetWgs workgroups plus one per (request, kv head) for the rounding: the
     // parts are never shorter than work / kRowTargetWgs (the waves' block-id registers bound
@@ -1080,12 +1110,12 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
     const int min_wave_tokens = max_row_len <= EDGERAG_ROW_SHORT_CTX
                                     ? EDGERAG_ROW_MIN_WAVE_TOKENS_SHORT
                                     : kRowMinWaveTokens;
-    const int64_t min_part = int64_t(kRowPartWaves) * round_up(min_wave_tokens, block_size);
+    const int64_t min_part = int64_t(part_waves) * round_up(min_wave_tokens, block_size);
     const int64_t want = (work + kRowTargetWgs - 1) / kRowTargetWgs;
-    const int64_t cap = int64_t(kRowPartWaves) * kMaxSplitBlocks * block_size;
+    const int64_t cap = int64_t(part_waves) * kMaxSplitBlocks * block_size;
     wg_part = std::min(cap, std::max(min_part, round_up(want, block_size)));
     wg_rows = true;
-    row_waves = kRowPartWaves;
+    row_waves = part_waves;
     // The parts write their partials to S fixed slots per (token, q head), the unused ones
     // marked empty, so that a merge addresses every partial from its thread index alone and
     // needs one round trip (attn_combine_slots_kernel). S (a power of two) covers the parts
@@ -1103,7 +1133,7 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
              (row_items <= kPlanCUs ||
               (row_items <= EDGERAG_ROW_WG_MAX_ITEMS && max_row_len <= EDGERAG_ROW_WG_SHORT))) {
     wg_rows = true;
-    row_waves = kRowWgWaves;
+    row_waves = full_waves;
   } else if (wg_capable && EDGERAG_ROW_WG_LONG) {
     wg_part = part_cap;
     wg_rows = true;
@@ -1304,7 +1334,8 @@ extern "C" int64_t edgerag_attn_fixed_row_items(int32_t max_reqs, int32_t n_kv_h
   const int64_t part_cap = int64_t(kRowWgWaves) * round_up(wave_cap, block_size);
   const int64_t per_req = std::max<int64_t>(1, (int64_t(max_context) + part_cap - 1) / part_cap);
   // Few-row parts: at most kRowTargetWgs + rh, or parts of the block-id cap when that binds.
-  const int64_t small_cap = int64_t(kRowPartWaves) * kMaxSplitBlocks * block_size;
+  const int64_t small_cap =
+      int64_t(std::min(kRowPartWaves, kGqaWaves)) * kMaxSplitBlocks * block_size;
   const int64_t per_req_small =
       std::max<int64_t>(1, (int64_t(max_context) + small_cap - 1) / small_cap);
   return std::max<int64_t>(

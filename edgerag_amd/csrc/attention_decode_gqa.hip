@@ -1,0 +1,468 @@
+// Decode rows of grouped-query attention on CDNA4 matrix cores (fp16 and bf16, head_dim 64 and 128).
+//
+// A row item is (request, kv head, keys) with 2 to 8 query vectors (new tokens x heads of the
+// group). The VALU kernel (attn_decode_kernel) spends 2 D operations per key, value and query
+// vector, so past one vector its time goes to arithmetic instead of to the stream of K and V. Here
+// a wave takes 32 keys a step:
+//   * S^T = K Q^T with v_mfma_f32_16x16x32: K goes from the pool to the A operand in registers
+//     (lane (key, g = lane / 16) loads dims 32 ks + 8 g .. + 7); Q is held as B, the up to 8
+//     vectors in columns 0-7 and again in 8-15.
+//   * softmax in the log2 domain, the reference max raised lazily (when a score beats it by 2^8).
+//   * O^T += V^T P^T with the same MFMA. Probabilities keep 16 + bits: columns 0-7 hold p rounded to
+//     the 16-bit type, columns 8-15 what the rounding left, and the two halves of O add up at the
+//     end, so the split costs no extra MFMA. V goes from the pool straight into a buffer of the
+//     wave in LDS (no staging registers) and is read transposed (ds_read_b64_tr_b16).
+// The next step's K (registers) and V (the other LDS buffer) are in flight while a step is
+// computed; waves do not wait for each other before the merge. Items are run as attn_decode_kernel
+// runs them: one wave per KV split, or a workgroup whose waves split the item's keys and merge in
+// LDS. A fused append stores the item's new rows to their slots first and reads them back.
+//
+// Bound by the K/V stream at large batches (bf16 32/8 heads of 128, 48 requests of 256-8,192
+// tokens, 870 MB: 213 -> 159 us, 4.1 -> 5.5 TB/s), by the chain of one wave's steps in small ones (one
+// request of 2,048 tokens 18.0 -> 9.6 us, 32 requests with 9/3 heads of 64 44.8 -> 25.2 us).
+#include "attention_merge.h"
+#include "attention_plan.h"
+
+namespace edgerag {
+namespace {
+
+using namespace plan;
+
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kVecs = 8;             // query vectors of an item
+constexpr int kKeys = 32;            // keys per step: two 16-key MFMA tiles
+constexpr float kRescaleLog2 = 8.f;
+constexpr uint32_t kOutOfRange = 0xFFFFF000u;
+
+// Cache policy of the K and V loads: non-temporal, a launch reads each byte once (48 requests,
+// 870 MB: 171 -> 159 us; batches small enough to stay in the last-level cache between launches,
+// which a model's layers do not, lose 2 to 4%).
+constexpr int kStream = 2;
+
+struct Slice {
+  const void* base;
+  uint32_t bytes;
+};
+__device__ __forceinline__ u32x4 load_slice(Slice s, uint32_t off) {
+  return __builtin_bit_cast(
+      u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                 __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(s.base), 0, s.bytes,
+                                                   0x00020000),
+                 off, 0, kStream));
+}
+// 16 bytes a lane from byte offset `off` of the slice (zeros past its end) to dst + 16 lane in LDS.
+__device__ __forceinline__ void load_lds16(Slice s, char* dst, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(s.base), 0, s.bytes, 0x00020000),
+      (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, kStream);
+}
+
+template <typename T>
+struct Elem;
+template <>
+struct Elem<f16> {
+  typedef h8 v8;
+  static __device__ __forceinline__ f32x4 mfma(v8 a, v8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t round2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, h2{_Float16(a), _Float16(b)});
+  }
+  static __device__ __forceinline__ float lo(uint32_t w) {
+    return float(__builtin_bit_cast(h2, w)[0]);
+  }
+  static __device__ __forceinline__ float hi(uint32_t w) {
+    return float(__builtin_bit_cast(h2, w)[1]);
+  }
+};
+template <>
+struct Elem<bf16> {
+  typedef b8 v8;
+  static __device__ __forceinline__ f32x4 mfma(v8 a, v8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t round2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, b2{__bf16(a), __bf16(b)});
+  }
+  static __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
+  static __device__ __forceinline__ float hi(uint32_t w) {
+    return __uint_as_float(w & 0xFFFF0000u);
+  }
+};
+
+// max / sum over the four lanes that differ in lane / 16.
+__device__ __forceinline__ float groups_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float groups_sum(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+// v plus its value 8 lanes on in the same row of 16 (row_ror:8).
+__device__ __forceinline__ float add_half_row(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF,
+                                                        false));
+}
+
+// Slot of chunk c of key k in a V buffer row is c ^ v_swizzle(k): 32 lanes of a transposing read
+// take 32 bytes (2 chunks) of each of 8 consecutive rows, which must cover all 256 bytes of banks
+// (rows of head_dim 64 alternate between the two halves already).
+template <int D>
+__device__ __forceinline__ int v_swizzle(int key) {
+  return D == 64 ? ((key >> 1) & 3) << 1 : (key & 7) << 1;
+}
+
+// NW: waves per workgroup (1: one wave per item).
+template <typename T, int D, int NW>
+__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2)))
+void attn_decode_gqa_kernel(
+    const int32_t* __restrict__ plan, int32_t item_base, int32_t limit_word,
+    const int32_t* __restrict__ qsl, const int32_t* __restrict__ ctx,
+    const int32_t* __restrict__ block_tables, int64_t bt_stride, int32_t num_blocks,
+    int32_t block_size, const T* __restrict__ q, int64_t q_st, int64_t q_sh,
+    const T* kpool, const T* vpool, int32_t n_q_heads, int32_t n_kv_heads, float scale_log2,
+    T* __restrict__ out, int64_t o_st, int64_t o_sh, float2* __restrict__ part_ml,
+    float* __restrict__ part_acc, const T* __restrict__ nk, const T* __restrict__ nv,
+    int64_t n_st, int64_t n_sh, const int32_t* __restrict__ slots, T* kdst, T* vdst) {
+  using E = Elem<T>;
+  typedef typename E::v8 v8;
+  constexpr int kKs = D / 32, kDt = D / 16, kCh = D / 8;
+  constexpr int kKpi = kWave / kCh;        // keys a V load covers
+  constexpr int kVLoads = kKeys / kKpi;
+  constexpr int kBuf = kKeys * D * 2;      // bytes of a V buffer
+  static_assert(kVecs * D * 4 <= kBuf, "the merge reuses a wave's V buffer");
+  // Two arrays, not one with an index: a load into one is then known not to alias the other.
+  __shared__ __align__(16) char sv0[NW * kBuf], sv1[NW * kBuf];
+  __shared__ float sml[NW][kVecs][2];
+
+  const int64_t idx = int64_t(item_base) + blockIdx.x;
+  if (idx >= plan[limit_word]) return;
+  const int32_t* it = plan + kHeaderWords + idx * kItemWords;
+  const int r = it[I_REQ], h = it[I_HEAD], qb = it[I_QBEGIN], qc = it[I_QCOUNT];
+  int kb = it[I_KVBEGIN], ke = it[I_KVEND];
+  const int split = it[I_SPLIT];
+  const int32_t* rq = plan + plan[H_REQ_OFF] + r * kReqWords;
+  const int lane = threadIdx.x % kWave;
+  const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave)) : 0;
+  if constexpr (NW > 1) {
+    // This wave's part: equal parts of whole blocks, empty for waves past the end.
+    const int per = (ke - kb + NW - 1) / NW;
+    const int part = (per + block_size - 1) / block_size * block_size;
+    const int b0 = min(ke, kb + wave * part);
+    ke = min(ke, b0 + part);
+    kb = b0;
+  }
+  // Block ids of the wave's keys, one per lane.
+  const int nblk = (ke - kb + block_size - 1) / block_size;
+  int32_t my_blk = -1;
+  if (nblk > 0)
+    my_blk = block_tables[int64_t(r) * bt_stride + kb / block_size + min(lane, nblk - 1)];
+  const int nsplit = rq[R_NSPLIT], part_off = rq[R_PARTOFF], pstride = rq[R_PSTRIDE];
+  const int q0 = qsl[r], c = qsl[r + 1] - q0, L = ctx[r];
+  if (lane >= nblk || my_blk >= num_blocks) my_blk = -1;
+  const int n_rep = n_q_heads / n_kv_heads;
+  const int nvec = qc * n_rep;
+  const int g = lane / 16, col = lane % 16, vec = col % kVecs;
+  const bool low = col >= kVecs;  // this column holds the rounding rests of vector `vec`
+  const bool active = vec < nvec;
+  const int t = qb + (active ? vec / n_rep : 0);
+  const int hq = h * n_rep + (active ? vec % n_rep : 0);
+  const int lim = active ? L - c + (t - q0) : -1;
+  const int min_lim = L - c + (qb - q0);
+
+  const int64_t head_base = int64_t(h) * num_blocks * block_size;
+  const uint32_t head_bytes = uint32_t(int64_t(num_blocks) * block_size * D * 2);
+  const Slice ks{kpool + head_base * D, head_bytes}, vs{vpool + head_base * D, head_bytes};
+
+  if (nk != nullptr && ke > L - c && kb < ke) {
+    // The new rows among this wave's keys go to their slots, and are read back below (same wave,
+    // after the stores are done).
+    for (int pos = max(kb, L - c); pos < ke; ++pos) {
+      const int64_t tok = q0 + (pos - (L - c));
+      const int64_t slot = slots[tok];
+      if (lane < 2 * kCh && slot >= 0 && slot < int64_t(num_blocks) * block_size) {
+        const T* src = (lane < kCh ? nk : nv) + tok * n_st + int64_t(h) * n_sh + lane % kCh * 8;
+        T* dst = (lane < kCh ? kdst : vdst) + (head_base + slot) * D + lane % kCh * 8;
+        store16(dst, load16(src));
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+
+  v8 qop[kKs];
+  {
+    const T* qp = q + int64_t(t) * q_st + int64_t(hq) * q_sh + 8 * g;
+#pragma unroll
+    for (int s = 0; s < kKs; ++s)
+      qop[s] = active ? *reinterpret_cast<const v8*>(qp + 32 * s) : v8{};
+  }
+  f32x4 o[kDt];
+#pragma unroll
+  for (int dt = 0; dt < kDt; ++dt) o[dt] = f32x4{};
+  float m = -INFINITY, l = 0.f, nm = 0.f;
+
+  // The load cursor: block index and row in the block of the next 16-key tile.
+  int cur_blk = 0, cur_row = 0;
+  // Byte offset of row `key` of the tile at tile_row (invalid or past the split: out of range).
+  auto next_tile = [&](int& blk, int& row) {
+    blk = __builtin_amdgcn_readlane(my_blk, min(cur_blk, kWave - 1));
+    row = blk * block_size + cur_row;
+    cur_row += 16;
+    if (cur_row >= block_size) {
+      cur_row = 0;
+      ++cur_blk;
+    }
+  };
+  auto load_step = [&](int k0, u32x4 (&kr)[2][kKs], char* sv) {
+    int blk[2], row[2];
+    next_tile(blk[0], row[0]);
+    next_tile(blk[1], row[1]);
+#pragma unroll
+    for (int tl = 0; tl < 2; ++tl) {
+      const uint32_t off = blk[tl] >= 0 && k0 + 16 * tl + col < ke
+                               ? uint32_t(row[tl] + col) * uint32_t(D * 2) + uint32_t(16 * g)
+                               : kOutOfRange;
+#pragma unroll
+      for (int s = 0; s < kKs; ++s) kr[tl][s] = load_slice(ks, off + uint32_t(64 * s));
+    }
+#pragma unroll
+    for (int j = 0; j < kVLoads; ++j) {
+      const int tl = kKpi * j / 16;
+      const int key = kKpi * j + lane / kCh;  // in the step
+      const int chunk = (lane % kCh) ^ v_swizzle<D>(key);
+      const uint32_t off = blk[tl] >= 0 && k0 + key < ke
+                               ? uint32_t(row[tl] + key % 16) * uint32_t(D * 2) + uint32_t(16 * chunk)
+                               : kOutOfRange;
+      load_lds16(vs, sv + j * 1024, off);
+    }
+  };
+  auto read_v = [&](const char* sv, int dt) {
+    union {
+      s4 half[2];
+      v8 all;
+    } u;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int key = 16 * i + 4 * g + col / 4;
+      const int dim = 16 * dt + 4 * (col % 4);
+      u.half[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (__attribute__((address_space(3))) s4*)(sv + key * (D * 2) +
+                                                  16 * ((dim / 8) ^ v_swizzle<D>(key)) +
+                                                  2 * (dim % 8)));
+    }
+    return u.all;
+  };
+  auto step = [&](int k0, const u32x4 (&kr)[2][kKs], const char* sv) {
+    f32x4 s[2] = {};
+#pragma unroll
+    for (int n = 0; n < kKs; ++n)
+#pragma unroll
+      for (int tl = 0; tl < 2; ++tl)
+        s[tl] = E::mfma(__builtin_bit_cast(v8, kr[tl][n]), qop[n], s[tl]);
+    // Register i of tile tl is key 16 tl + 4 g + i.
+    const bool bad = __any(my_blk < 0 && lane < nblk);
+#pragma unroll
+    for (int tl = 0; tl < 2; ++tl)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[tl][i] = __builtin_fmaf(s[tl][i], scale_log2, nm);
+    if (k0 + kKeys - 1 > min_lim || k0 + kKeys > ke || bad) {
+      const int vis_end = min(ke, lim + 1) - k0 - 4 * g;
+#pragma unroll
+      for (int tl = 0; tl < 2; ++tl) {
+        const bool gone =
+            bad && __builtin_amdgcn_readlane(
+                       my_blk, min((k0 - kb + 16 * tl) / block_size, kWave - 1)) < 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (gone || 16 * tl + i >= vis_end) s[tl][i] = -INFINITY;
+      }
+    }
+    float tmax = s[0][0];
+#pragma unroll
+    for (int tl = 0; tl < 2; ++tl)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[tl][i]);
+    tmax = groups_max(tmax);
+    const bool first = m == -INFINITY;
+    const bool up = first ? tmax != -INFINITY : tmax > kRescaleLog2;
+    if (__any(up)) {
+      const float shift = up ? tmax : 0.f;
+      const float alpha = first ? (up ? 0.f : 1.f) : exp2_fast(-shift);
+      if (up) m = first ? tmax : m + tmax;
+      nm = m == -INFINITY ? 0.f : -m;
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt) o[dt] *= alpha;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[0][i] -= shift;
+        s[1][i] -= shift;
+      }
+    }
+    u32x4 pw;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float p0 = exp2_fast(s[w / 2][2 * (w % 2)]), p1 = exp2_fast(s[w / 2][2 * (w % 2) + 1]);
+      l += p0 + p1;
+      const uint32_t head = E::round2(p0, p1);
+      const uint32_t rest = E::round2(p0 - E::lo(head), p1 - E::hi(head));
+      pw[w] = low ? rest : head;
+    }
+    const v8 p = __builtin_bit_cast(v8, pw);
+    // This step's V has landed when only the loads of the next step, issued after it, are left.
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kKs + kVLoads) : "memory");
+#pragma unroll
+    for (int dt = 0; dt < kDt; ++dt) o[dt] = E::mfma(read_v(sv, dt), p, o[dt]);
+  };
+
+  char* const buf0 = sv0 + wave * kBuf;
+  char* const buf1 = sv1 + wave * kBuf;
+  u32x4 k0r[2][kKs], k1r[2][kKs];
+  if (kb < ke) load_step(kb, k0r, buf0);
+  for (int k0 = kb; k0 < ke; k0 += 2 * kKeys) {
+    load_step(k0 + kKeys, k1r, buf1);
+    issue_fence();
+    step(k0, k0r, buf0);
+    if (k0 + kKeys >= ke) break;
+    load_step(k0 + 2 * kKeys, k0r, buf0);
+    issue_fence();
+    step(k0 + kKeys, k1r, buf1);
+  }
+  // Loads past the keys may still be on their way into this wave's buffers.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  l = groups_sum(l);
+#pragma unroll
+  for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[dt][i] = add_half_row(o[dt][i]);
+
+  // Register i of O tile dt holds dim 16 dt + 4 g + i of vector `vec`.
+  const int64_t row0 = int64_t(part_off) + (int64_t(t - q0) * n_q_heads + hq) * pstride;
+  if constexpr (NW == 1) {
+    if (!active || low) return;
+    if (nsplit == 1) {
+      const float inv = 1.f / fmaxf(l, 1.17549435e-38f);
+      T* op = out + int64_t(t) * o_st + int64_t(hq) * o_sh;
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) op[16 * dt + 4 * g + i] = from_f32<T>(o[dt][i] * inv);
+    } else {
+      if (g == 0) part_ml[row0 + split] = make_float2(m, l);
+      float* pa = part_acc + (row0 + split) * D;
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt)
+        *reinterpret_cast<f32x4*>(pa + 16 * dt + 4 * g) = o[dt];
+    }
+  } else {
+    // The waves' (m, l, O) meet in their own V buffers; the workgroup merges and writes.
+    float* acc0 = reinterpret_cast<float*>(buf0);
+    if (active && !low) {
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt)
+        *reinterpret_cast<f32x4*>(acc0 + vec * D + 16 * dt + 4 * g) = o[dt];
+      if (g == 0) {
+        sml[wave][vec][0] = m;
+        sml[wave][vec][1] = l;
+      }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < nvec * D; e += NW * kWave) {
+      const int v = e / D, d = e % D;
+      float mx = -INFINITY, lsum = 0.f, a = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) mx = fmaxf(mx, sml[w][v][0]);
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float mw = sml[w][v][0];
+        const float wgt = mw == -INFINITY ? 0.f : exp2_fast(mw - mx);
+        lsum = __builtin_fmaf(wgt, sml[w][v][1], lsum);
+        a = __builtin_fmaf(wgt, reinterpret_cast<const float*>(sv0 + w * kBuf)[v * D + d], a);
+      }
+      const int tv = qb + v / n_rep, hv = h * n_rep + v % n_rep;
+      if (pstride == 1) {
+        out[int64_t(tv) * o_st + int64_t(hv) * o_sh + d] =
+            from_f32<T>(a * (1.f / fmaxf(lsum, 1.17549435e-38f)));
+      } else {
+        const int64_t rv = int64_t(part_off) + (int64_t(tv - q0) * n_q_heads + hv) * pstride;
+        if (d == 0) part_ml[rv + split] = make_float2(mx, lsum);
+        // The last part marks the unused slots of a slotted row empty.
+        if (split == nsplit - 1 && nsplit + d < pstride)
+          part_ml[rv + nsplit + d] = make_float2(-INFINITY, 0.f);
+        part_acc[(rv + split) * D + d] = a;
+      }
+    }
+  }
+}
+
+template <typename T, int D, int NW>
+void launch(const AttnLaunch& a, int base, int count, int limit_word) {
+  hipLaunchKernelGGL((attn_decode_gqa_kernel<T, D, NW>), dim3(count), dim3(NW * kWave), 0, a.s,
+                     a.plan, base, limit_word, a.qsl, a.ctx, a.bt, a.bt_stride, a.nb, a.bs,
+                     static_cast<const T*>(a.q), a.q_st, a.q_sh, static_cast<const T*>(a.kp),
+                     static_cast<const T*>(a.vp), a.hq, a.hkv, a.scale_log2,
+                     static_cast<T*>(a.out), a.o_st, a.o_sh, a.ml, a.pacc,
+                     static_cast<const T*>(a.nk), static_cast<const T*>(a.nv), a.n_st, a.n_sh,
+                     a.slots, static_cast<T*>(const_cast<void*>(a.kp)),
+                     static_cast<T*>(const_cast<void*>(a.vp)));
+}
+
+// Waves of a workgroup row this kernel is built for: those the planner gives rows of the head_dim.
+bool row_waves_built(int32_t head_dim, int waves) {
+  return waves == 0 || (head_dim == 64 ? waves == 8 || waves == 16 : waves == kGqaWaves);
+}
+
+template <typename T, int D>
+void launch_waves(const AttnLaunch& a, int base, int count, int limit_word, int waves) {
+  if (waves == 0) {
+    launch<T, D, 1>(a, base, count, limit_word);
+  } else if constexpr (D == 64) {
+    if (waves == 8) launch<T, D, 8>(a, base, count, limit_word);
+    else launch<T, D, 16>(a, base, count, limit_word);
+  } else {
+    launch<T, D, kGqaWaves>(a, base, count, limit_word);
+  }
+}
+
+}  // namespace
+
+bool decode_gqa_shape(int32_t dtype, int32_t head_dim, int vecs, int32_t block_size) {
+  return (dtype == EDGERAG_F16 || dtype == EDGERAG_BF16) && (head_dim == 64 || head_dim == 128) &&
+         vecs >= 2 && vecs <= kVecs && block_size % 16 == 0;
+}
+
+bool decode_gqa_supported(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int vecs,
+                          int waves) {
+  return decode_gqa_shape(dtype, head_dim, vecs, a.bs) && row_waves_built(head_dim, waves) &&
+         int64_t(a.nb) * a.bs * head_dim * 2 < int64_t(kOutOfRange);
+}
+
+void launch_decode_gqa(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int base, int count,
+                       int limit_word, int waves) {
+  const bool half = dtype == EDGERAG_F16;
+  if (head_dim == 64) {
+    if (half) launch_waves<f16, 64>(a, base, count, limit_word, waves);
+    else launch_waves<bf16, 64>(a, base, count, limit_word, waves);
+  } else {
+    if (half) launch_waves<f16, 128>(a, base, count, limit_word, waves);
+    else launch_waves<bf16, 128>(a, base, count, limit_word, waves);
+  }
+}
+
+}  // namespace edgerag

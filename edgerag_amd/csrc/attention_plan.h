@@ -95,6 +95,15 @@ bool prefill_tile_shape(int32_t dtype, int32_t head_dim);
 // Whether a pool of this size can use it (buffer-resource addressing).
 bool prefill_tiles_supported(int32_t num_blocks, int32_t block_size, int32_t head_dim);
 
+constexpr int kGqaWaves = 4;  // waves of a workgroup row of the GQA kernel at head_dim 128
+// Decode rows with 2 to 8 query vectors on MFMA (attention_decode_gqa.hip): fp16 and bf16, head_dim
+// 64 and 128, one wave per item or workgroup rows.
+// Whether the kernel is built for the shape, and whether it takes this launch.
+bool decode_gqa_shape(int32_t dtype, int32_t head_dim, int vecs, int32_t block_size);
+bool decode_gqa_supported(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int vecs,
+                          int waves);
+void launch_decode_gqa(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int base, int count,
+                       int limit_word, int waves);
 // Prefill tiles in fp32 (attention_prefill_f32.hip), head_dim 64 and 128: 16 or 32 virtual rows.
 void launch_prefill_f32(const AttnLaunch& a, int32_t head_dim, int rows, int item_base, int count);
 bool prefill_f32_supported(int32_t num_blocks, int32_t block_size, int32_t head_dim);

@@ -446,6 +446,50 @@ def test_wide_prefill_tiles_at_other_block_sizes(device, dtype, d, reqs, bs) -> 
             torch.testing.assert_close(got[r * c : (r + 1) * c, hq], ref, **tol)
 
 
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 64),
+                                     (torch.float16, 128), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("n_q,n_kv,reqs,bs", [(4, 2, 9, 16), (9, 3, 9, 48), (16, 2, 9, 16),
+                                              (32, 32, 9, 32), (64, 32, 9, 16)])
+@pytest.mark.parametrize("split_rows", [False, True])
+def test_grouped_decode_rows(device, dtype, d, n_q, n_kv, reqs, bs, split_rows) -> None:
+    """Decode rows of 2 to 8 query vectors on the matrix cores: contexts around the 16-key tile and
+    the 32-key step, one- and two-token requests, parts, whole-context workgroups and KV splits,
+    block sizes that hold several tiles, NaN past every context and one invalid block, against
+    the float64 softmax (the tolerances of the wide prefill tiles)."""
+    g = seeded(d + n_q + bs)
+    rep = n_q // n_kv
+    lens = [1, 15, 17, 32, 33, 49, 300, 1100, 2100][:reqs]
+    q_lens = [1] * reqs
+    q_lens[4] = 2 if rep < 5 else 1
+    if n_q == n_kv:  # one query head a group: the rows of two tokens bring the second vector
+        q_lens = [1, 2] * reqs
+        q_lens = [min(c, L) for c, L in zip(q_lens, lens)]
+    nbs = [-(-L // bs) for L in lens]
+    kp, vp = (torch.randn(n_kv, sum(nbs), bs, d, generator=g).to(dtype) for _ in range(2))
+    perm = torch.randperm(sum(nbs), generator=g).split(nbs)
+    bt = np.full((reqs, max(nbs)), -1, np.int32)
+    for r, ids in enumerate(perm):
+        bt[r, : nbs[r]] = ids.numpy()
+        if lens[r] % bs:
+            kp[:, ids[-1], lens[r] % bs :] = vp[:, ids[-1], lens[r] % bs :] = float("nan")
+    bt[6, 2] = -1  # an invalid block inside a context is not read
+    qsl = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    q = torch.randn(int(qsl[-1]), n_q, d, generator=g).to(dtype)
+    plan, _ = kernels.plan_attention(qsl, np.asarray(lens, np.int32), bt, n_q, n_kv, d, bs, dtype,
+                                     device, split_rows=split_rows)
+    got = kernels.paged_attention(q.to(device), kp.to(device), vp.to(device), plan,
+                                  d**-0.5).cpu().double()
+    u = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-11
+    for r, (L, c) in enumerate(zip(lens, q_lens)):
+        keep = torch.ones(nbs[r] * bs, dtype=torch.bool)[:L]
+        if r == 6:
+            keep[2 * bs : 3 * bs] = False
+        for h in (0, n_q - 1):
+            k, v = (p[h // rep, perm[r]].reshape(-1, d)[:L][keep].float() for p in (kp, vp))
+            ref = oa.attention_f64(q[qsl[r] : qsl[r + 1], h].float(), k, v, len(k) - c, d**-0.5)
+            torch.testing.assert_close(got[qsl[r] : qsl[r + 1], h], ref, rtol=2 * u, atol=u / 64)
+
+
 def test_cfg2_shape_decode_batch_fp16(device) -> None:
     """BASELINE config 2 at full shape: 32 decodes, L ~ U[256, 7472], 32/32 heads, d 64,
     16,384-block pool (1 GiB per pool), seeded-shuffled tables."""
