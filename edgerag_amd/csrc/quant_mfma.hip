@@ -901,6 +901,23 @@ __device__ __forceinline__ void gemm_store_x(const GemmStage<C>& st, int i, _Flo
 // SPLIT: blockIdx.z is one of gridDim.z equal k ranges (split K). The workgroup writes its fp32
 // partial tile to sk.part and stops; qlinear_split_reduce_kernel, the next launch on the stream,
 // adds the partials in split order and applies the epilogue.
+// Tile (tx, ty) of this workgroup of a launch of 256x256 tiles. Workgroups go to the 8 XCDs in turn, each
+// with an L2 of its own: XCD c takes the c-th contiguous run of an order that walks kTileGroup rows
+// of tiles at a time, so that the 32 tiles an XCD works on together are 8 x 4, not 4 x 8 or worse:
+// they share weight and (twice as many bytes a row) activation rows. M = 2,048, 2048 -> 8192:
+// 92.6 -> 76.5 us, where the plain order gives an XCD all 8 activation tiles; 2048 -> 16384, whose
+// plain order is 8 x 4 already, unchanged. (128x128 tiles measured no gain, 256 of them a loss.)
+constexpr int kTileGroup = 4;
+__device__ __forceinline__ void xcd_tile(int& tx, int& ty) {
+  const int gx = gridDim.x, gy = gridDim.y;
+  const int id0 = blockIdx.y * gx + blockIdx.x, per = gx * gy / 8, more = gx * gy % 8;
+  const int xcd = id0 % 8;  // has per tiles, the first `more` XCDs one more
+  const int id = xcd * per + min(xcd, more) + id0 / 8;
+  const int y0 = id / (kTileGroup * gx) * kTileGroup, rows = min(kTileGroup, gy - y0);
+  tx = (id - y0 * gx) / rows;
+  ty = y0 + (id - y0 * gx) % rows;
+}
+
 // By value to every tiled-GEMM launch: the split partials, or the RoPE epilogue's operands.
 struct GemmArgs {
   float* part;  // [tiles][splits][BN * BM] fp32 partial tiles
@@ -933,7 +950,9 @@ __global__ __launch_bounds__(NTH, EDGERAG_GEMM_MIN_WG) void qlinear_gemm_kernel(
   __shared__ __attribute__((aligned(16))) _Float16 sx[2][BM * kLdsRow];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wn = wave % C::NWN, wm = wave / C::NWN;
-  const int nb = blockIdx.x * BN, mb = blockIdx.y * BM;
+  int tx = blockIdx.x, ty = blockIdx.y;
+  if constexpr (BN == 256) xcd_tile(tx, ty);
+  const int nb = tx * BN, mb = ty * BM;
   const int64_t row_bytes = BITS == 8 ? k : k / 2;
   const int groups = k / g;
 
@@ -1658,6 +1677,20 @@ void dispatch_stream_swiglu(const f16* x, int64_t xs, int32_t m, int32_t k, cons
     launch_stream_k<1, 2, 4, kEpiSwiglu>(x, xs, m, k, packed, scales, bias, n, y, ys, s);
 }
 
+// 256x256 tiles (512 threads, two waves per SIMD; an operand read from LDS feeds twice the MFMAs of
+// a 128x128 tile) where they are faster than 128x128. Modelled in rounds over the 256 CUs: a full
+// round of 256x256 tiles takes 3.3 rounds of 128x128 ones, a last, partial round 2.4 to 3.3.
+// Measured, 128x128 / 256x256 tiles, us: INT8 2,048 rows 2048 -> 16384 184 / 156, 2048 -> 8192 91 /
+// 76, 1,024 rows 2048 -> 16384 93 / 77, 512 rows 48 / 61; INT4 2,048 rows 4608 -> 4608 157 / 131.
+// Sums run in the same order: the same bits.
+bool gemm_tiles_256(int32_t m, int32_t n) {
+  const int64_t t256 = int64_t((n + 255) / 256) * ((m + 255) / 256);
+  const int64_t t128 = int64_t((n + 127) / 128) * ((m + 127) / 128);
+  const int64_t last = t256 % 256;
+  const int64_t cost256 = t256 / 256 * 33 + (last > 0 ? 24 + last * 9 / 256 : 0);
+  return cost256 < (t128 + 255) / 256 * 10;
+}
+
 template <int BITS>
 void dispatch(const f16* x, int64_t xs, int32_t m, int32_t k, const uint8_t* packed,
               const f16* scales, const f16* bias, int32_t n, int32_t g, f16* y, int64_t ys,
@@ -1689,6 +1722,10 @@ void dispatch(const f16* x, int64_t xs, int32_t m, int32_t k, const uint8_t* pac
     dispatch<BITS>(x, xs, m - rem, k, packed, scales, bias, n, g, y, ys, s);
     dispatch<BITS>(x + int64_t(m - rem) * xs, xs, rem, k, packed, scales, bias, n, g,
                    y + int64_t(m - rem) * ys, ys, s);
+    return;
+  }
+  if (gemm_tiles_256(m, n)) {
+    launch_gemm<BITS, 256, 256, 512, 2>(x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
     return;
   }
   // Tiles: the largest whose grid still covers the 256 CUs.

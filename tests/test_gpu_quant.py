@@ -648,3 +648,27 @@ def test_quant_state_dict_round_trips_through_safetensors(device, tmp_path, bits
     assert torch.equal(c.packed, a.packed) and torch.equal(c.scales, a.scales)
     expected = oq.quant_linear_reference(x.cpu(), packed, scales, bias, k, oq.QuantConfig(cfg.group_size, bits))
     torch.testing.assert_close(c(x).float().cpu(), expected, **LINEAR_TOL)
+
+
+@pytest.mark.parametrize("bits,k,g", [(8, 64, 64), (8, 320, 320), (8, 384, 32), (4, 128, 32),
+                                      (4, 640, 128)])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_wide_gemm_tiles_equal_the_narrow_ones(device, bits, k, g, with_bias) -> None:
+    """Shapes that take 256x256 tiles (ragged in rows and columns, one and an odd number of 64-k
+    steps, group scales): every output has the bits of the same rows run 200 at a time, which
+    take 128x128 tiles (a row's sum does not depend on the tile), and is within the linear
+    tolerance of dequantise-then-matmul."""
+    gen = torch.Generator(device=device).manual_seed(bits * k + g)
+    m, n = 1000, 16300
+    w = torch.randn(n, k, generator=gen, device=device) * 0.02
+    packed, scales = kernels.quantize(w, bits, g)
+    bias = torch.randn(n, generator=gen, device=device).half() if with_bias else None
+    x = torch.randn(m, k, generator=gen, device=device).half()
+    got = kernels.quant_linear(x, packed, scales, bias, k, n, bits, g, split_k=False)
+    rows = [kernels.quant_linear(x[i : i + 200], packed, scales, bias, k, n, bits, g,
+                                 split_k=False) for i in range(0, m, 200)]
+    assert torch.equal(got, torch.cat(rows))
+    ref = x.float() @ kernels.dequantize(packed, scales, k, bits, g).float().t()
+    if with_bias:
+        ref += bias.float()
+    torch.testing.assert_close(got.float(), ref, rtol=1e-2, atol=1e-2 * float(ref.std()))
