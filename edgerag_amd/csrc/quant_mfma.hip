@@ -892,17 +892,8 @@ __device__ __forceinline__ void gemm_store_x(const GemmStage<C>& st, int i, _Flo
   *reinterpret_cast<uint4*>(sx + lds_off(xr, xc0 + i)) = st.x[i];
 }
 
-// y[M, N] = x . W^T for one BN x BM tile of y^T. Waves form a 2 x 2 grid; wave (wn, wm) owns
-// rows [wn BN/2, +BN/2) of the weight tile and [wm BM/2, +BM/2) of the activation tile, as
-// TN x TM 32x32 MFMA tiles. Operand lane layout of v_mfma_f32_32x32x16_f16: lane l reads row
-// l % 32, k chunk 2 ks + l / 32 of a 16-k step; accumulator register i of lane l holds
-// row 8 (i / 4) + 4 (l / 32) + i % 4 of A (weight row) and column l % 32 (activation row).
-// PC: per-channel INT8 (one scale per weight row), applied to the fp32 sums.
-// SPLIT: blockIdx.z is one of gridDim.z equal k ranges (split K). The workgroup writes its fp32
-// partial tile to sk.part and stops; qlinear_split_reduce_kernel, the next launch on the stream,
-// adds the partials in split order and applies the epilogue.
-// Tile (tx, ty) of this workgroup of a launch of 256x256 tiles. Workgroups go to the 8 XCDs in turn, each
-// with an L2 of its own: XCD c takes the c-th contiguous run of an order that walks kTileGroup rows
+// Tile (tx, ty) of this workgroup of a launch of 256x256 tiles. Workgroups go to the 8 XCDs in
+// turn, each with an L2 of its own: XCD c takes the c-th contiguous run of an order that walks kTileGroup rows
 // of tiles at a time, so that the 32 tiles an XCD works on together are 8 x 4, not 4 x 8 or worse:
 // they share weight and (twice as many bytes a row) activation rows. M = 2,048, 2048 -> 8192:
 // 92.6 -> 76.5 us, where the plain order gives an XCD all 8 activation tiles; 2048 -> 16384, whose
@@ -918,6 +909,15 @@ __device__ __forceinline__ void xcd_tile(int& tx, int& ty) {
   ty = y0 + (id - y0 * gx) % rows;
 }
 
+// y[M, N] = x . W^T for one BN x BM tile of y^T. Waves form a 2 x 2 grid; wave (wn, wm) owns
+// rows [wn BN/2, +BN/2) of the weight tile and [wm BM/2, +BM/2) of the activation tile, as
+// TN x TM 32x32 MFMA tiles. Operand lane layout of v_mfma_f32_32x32x16_f16: lane l reads row
+// l % 32, k chunk 2 ks + l / 32 of a 16-k step; accumulator register i of lane l holds
+// row 8 (i / 4) + 4 (l / 32) + i % 4 of A (weight row) and column l % 32 (activation row).
+// PC: per-channel INT8 (one scale per weight row), applied to the fp32 sums.
+// SPLIT: blockIdx.z is one of gridDim.z equal k ranges (split K). The workgroup writes its fp32
+// partial tile to sk.part and stops; qlinear_split_reduce_kernel, the next launch on the stream,
+// adds the partials in split order and applies the epilogue.
 // By value to every tiled-GEMM launch: the split partials, or the RoPE epilogue's operands.
 struct GemmArgs {
   float* part;  // [tiles][splits][BN * BM] fp32 partial tiles
@@ -1613,17 +1613,76 @@ void dispatch_stream_residual(const f16* x, int64_t xs, int32_t m, int32_t k,
   }
 }
 
+// 256x256 tiles (512 threads, two waves per SIMD; an operand read from LDS feeds twice the MFMAs of
+// a 128x128 tile) where they are faster than 128x128. Modelled in rounds over the 256 CUs: a full
+// round of 256x256 tiles takes 3.3 rounds of 128x128 ones, a last, partial round 2.4 to 3.3.
+// Measured, 128x128 / 256x256 tiles, us: INT8 2,048 rows 2048 -> 16384 184 / 156, 2048 -> 8192 91 /
+// 76, 1,024 rows 2048 -> 16384 93 / 77, 512 rows 48 / 61; INT4 2,048 rows 4608 -> 4608 157 / 131.
+// Sums run in the same order: the same bits.
+bool gemm_tiles_256(int32_t m, int32_t n) {
+  const int64_t t256 = int64_t((n + 255) / 256) * ((m + 255) / 256);
+  const int64_t t128 = int64_t((n + 127) / 128) * ((m + 127) / 128);
+  const int64_t last = t256 % 256;
+  const int64_t cost256 = t256 / 256 * 33 + (last > 0 ? 24 + last * 9 / 256 : 0);
+  return cost256 < (t128 + 255) / 256 * 10;
+}
+
+// The tile of the tiled GEMM: 64x64, 128x64, 128x128 (the largest whose grid covers the 256 CUs), or
+//   * 128x256 (512 threads: the 64x64 of a wave as in 128x128, two waves per SIMD, half the weight
+//     reads) where 128x128 tiles need a second round and 128x256 ones do not: 128x128 / 128x256, INT8,
+//     us: 512 rows 2048 -> 16384 45.4 / 42.8, 768 rows 2048 -> 6144 37.2 / 33.7, 1,024 rows 2048 ->
+//     8192 44.9 / 42.4, 4096 -> 6144 71.8 / 63.6, 2,048 rows 8192 -> 4096 159 / 142. A second round
+//     that is nearly empty costs little, and INT4 dequantises more a tile: 1,024 rows 4608 -> 4608,
+//     288 tiles, 80.7 / 86.4 (900 rows), 1,536 rows, 432 tiles, 95.2 / 91.1.
+//   * 128x128 for less than one round, where 128x64 tiles need a second: 128x64 / 128x128, us: 519
+//     rows 2048 -> 6144 25.1 / 23.0, 560 rows 2048 -> 4096 23.4 / 21.7, 1,536 rows 2048 -> 2048 24.9
+//     / 22.7. Only for INT8 layers of up to 12 M codes: a round of fewer, larger workgroups has fewer
+//     loads in flight, and past that the weights take longer (4096 -> 4096 at 640 rows 44.2 / 46.3,
+//     2048 -> 8192 at 384 rows 25.0 / 25.6; INT4 1152 -> 3456 at 640 rows 18.6 / 19.4).
+// Every tile sums in the same order: the same bits.
+enum class GemmTile { k64, k128x64, k128, k128x256, k256 };
+
+inline int64_t gemm_tiles(int32_t m, int32_t n, int bm, int bn) {
+  return int64_t((n + bn - 1) / bn) * ((m + bm - 1) / bm);
+}
+
+GemmTile gemm_tile(int32_t m, int32_t k, int32_t n, int bits) {
+  constexpr int64_t kCUs = EDGERAG_GEMM_TARGET_WGS, kCodes128 = int64_t(12) << 20;
+  if (gemm_tiles_256(m, n)) return GemmTile::k256;
+  const int64_t t128 = gemm_tiles(m, n, 128, 128), t128x64 = gemm_tiles(m, n, 64, 128);
+  if (t128 > (bits == 8 ? kCUs : kCUs * 5 / 4) && gemm_tiles(m, n, 256, 128) <= kCUs)
+    return GemmTile::k128x256;
+  if (t128 >= kCUs) return GemmTile::k128;
+  if (t128x64 < kCUs) return GemmTile::k64;
+  return bits == 8 && t128x64 > kCUs && int64_t(n) * k <= kCodes128 ? GemmTile::k128
+                                                                    : GemmTile::k128x64;
+}
+
+// Rows past whole 64-row tiles (the decode tokens packed after a prefill chunk) that run on the
+// streaming (or skinny) path as a second launch: at most 16, and only where the tiles then take
+// another kind or fewer rounds over the CUs, since the second launch reads all weights again
+// (2048 -> 8192, 519 rows: 31.8 against 34.8 us in one launch; but 900 rows, the same rounds with
+// and without the last four, 46.2 against 40.6; 2048 -> 16384, 200 rows 32.6 against 24.5). 128x64
+// tiles (up to three workgroups per CU) take an extra row at almost no cost. 64x64 tiles always
+// pass them on, as the workspace route does (2048 -> 2048, 519 rows: 14.7 against 15.8).
+int gemm_remainder(int32_t m, int32_t k, int32_t n, int bits) {
+  const int rem = m % 64;
+  if (rem == 0 || rem > 16 || m - rem < 128) return 0;
+  const GemmTile tile = gemm_tile(m, k, n, bits);
+  if (tile == GemmTile::k64) return rem;
+  if (tile == GemmTile::k128x64) return 0;
+  if (gemm_tile(m - rem, k, n, bits) != tile)
+    return tile == GemmTile::k128 && gemm_tiles(m, n, 128, 128) <= EDGERAG_GEMM_TARGET_WGS ? 0 : rem;
+  const int bm = tile == GemmTile::k128 ? 128 : 256, bn = tile == GemmTile::k256 ? 256 : 128;
+  auto rounds = [&](int32_t rows) {
+    return (gemm_tiles(rows, n, bm, bn) + EDGERAG_GEMM_TARGET_WGS - 1) / EDGERAG_GEMM_TARGET_WGS;
+  };
+  return rounds(m) > rounds(m - rem) ? rem : 0;
+}
+
 // The streaming shapes with two row tiles of one k-slice: the only ones the SwiGLU form covers.
 // dispatch_stream picks exactly these for the same (M, K, N), so the fused launch computes the
 // same gate and up bits as the plain one.
-// The tiled GEMM's tile for M x N: the largest whose grid still covers the 256 CUs, 128x128,
-// else 128x64 (this test), else 64x64.
-inline bool gemm_tiles_128x64(int32_t m, int32_t n) {
-  const int64_t tn = (n + 127) / 128;
-  return tn * ((m + 127) / 128) < EDGERAG_GEMM_TARGET_WGS &&
-         tn * ((m + 63) / 64) >= EDGERAG_GEMM_TARGET_WGS;
-}
-
 bool stream_swiglu_shape(int32_t m, int32_t k, int32_t n) {
   return m <= EDGERAG_STREAM_MAX_M && stream_slices(m, k, n) == 1 && n % 2 == 0 &&
          (int64_t(n) + 15) / 16 >= EDGERAG_STREAM_NT2_TILES;
@@ -1635,11 +1694,9 @@ bool stream_swiglu_shape(int32_t m, int32_t k, int32_t n) {
 // streaming path goes to the streaming SwiGLU kernel.
 bool gemm_swiglu_shape(int32_t m, int32_t k, int32_t n) {
   if (m <= EDGERAG_SKINNY_MAX_M || n % 2 != 0 || k % kBK != 0) return false;
-  const int rem = m % 64;
-  if (rem > 0 && rem <= 16 && m - rem >= 128 && !gemm_tiles_128x64(m, n))
+  if (const int rem = gemm_remainder(m, k, n, 8))
     return gemm_swiglu_shape(m - rem, k, n) && stream_swiglu_shape(rem, k, n);
-  return int64_t((n + 127) / 128) * ((m + 127) / 128) >= EDGERAG_GEMM_TARGET_WGS ||
-         gemm_tiles_128x64(m, n);
+  return gemm_tile(m, k, n, 8) != GemmTile::k64;
 }
 
 void dispatch_stream_swiglu(const f16* x, int64_t xs, int32_t m, int32_t k, const uint8_t* packed,
@@ -1649,14 +1706,18 @@ void dispatch_stream_swiglu(const f16* x, int64_t xs, int32_t m, int32_t k, cons
 void dispatch_gemm_swiglu(const f16* x, int64_t xs, int32_t m, int32_t k, const uint8_t* packed,
                           const f16* scales, const f16* bias, int32_t n, f16* y, int64_t ys,
                           hipStream_t s) {
-  const int rem = m % 64;
-  if (rem > 0 && rem <= 16 && m - rem >= 128 && !gemm_tiles_128x64(m, n)) {
+  if (const int rem = gemm_remainder(m, k, n, 8)) {
     dispatch_gemm_swiglu(x, xs, m - rem, k, packed, scales, bias, n, y, ys, s);
     dispatch_stream_swiglu(x + int64_t(m - rem) * xs, xs, rem, k, packed, scales, bias, n,
                            y + int64_t(m - rem) * ys, ys, EpiArgs{}, s);
     return;
   }
-  if (int64_t((n + 127) / 128) * ((m + 127) / 128) >= EDGERAG_GEMM_TARGET_WGS)
+  const GemmTile tile = gemm_tile(m, k, n, 8);
+  // 256x256 tiles hold four 32-row tiles a wave, which the epilogue does not pair: 128x256 ones
+  // (2,048 rows 2048 -> 16384: 166 us on 128x128 tiles, 157 on these).
+  if (tile == GemmTile::k128x256 || tile == GemmTile::k256)
+    launch_gemm_swiglu<256, 512, 2>(x, xs, m, k, packed, scales, bias, n, y, ys, s);
+  else if (tile == GemmTile::k128)
     launch_gemm_swiglu<128, EDGERAG_GEMM_THREADS_128, EDGERAG_GEMM_STAGES_128>(
         x, xs, m, k, packed, scales, bias, n, y, ys, s);
   else
@@ -1675,20 +1736,6 @@ void dispatch_stream_swiglu(const f16* x, int64_t xs, int32_t m, int32_t k, cons
     launch_stream_k<1, 2, 2, kEpiSwiglu>(x, xs, m, k, packed, scales, bias, n, y, ys, s);
   else
     launch_stream_k<1, 2, 4, kEpiSwiglu>(x, xs, m, k, packed, scales, bias, n, y, ys, s);
-}
-
-// 256x256 tiles (512 threads, two waves per SIMD; an operand read from LDS feeds twice the MFMAs of
-// a 128x128 tile) where they are faster than 128x128. Modelled in rounds over the 256 CUs: a full
-// round of 256x256 tiles takes 3.3 rounds of 128x128 ones, a last, partial round 2.4 to 3.3.
-// Measured, 128x128 / 256x256 tiles, us: INT8 2,048 rows 2048 -> 16384 184 / 156, 2048 -> 8192 91 /
-// 76, 1,024 rows 2048 -> 16384 93 / 77, 512 rows 48 / 61; INT4 2,048 rows 4608 -> 4608 157 / 131.
-// Sums run in the same order: the same bits.
-bool gemm_tiles_256(int32_t m, int32_t n) {
-  const int64_t t256 = int64_t((n + 255) / 256) * ((m + 255) / 256);
-  const int64_t t128 = int64_t((n + 127) / 128) * ((m + 127) / 128);
-  const int64_t last = t256 % 256;
-  const int64_t cost256 = t256 / 256 * 33 + (last > 0 ? 24 + last * 9 / 256 : 0);
-  return cost256 < (t128 + 255) / 256 * 10;
 }
 
 template <int BITS>
@@ -1712,33 +1759,31 @@ void dispatch(const f16* x, int64_t xs, int32_t m, int32_t k, const uint8_t* pac
     }
     return;
   }
-  // A remainder of at most 16 rows past a whole number of 64-row tiles (the decode tokens packed
-  // after a prefill chunk) runs on the streaming (or skinny) path as a second launch, where an
-  // extra row of 128x128 or 64x64 tiles would be mostly empty. 128x64 tiles (up to three
-  // workgroups per CU) take the extra row at almost no cost, less than a second pass over the
-  // weights (2048->6144, M = 519: 28.1 against 33.5 us; M = 512: 28.2).
-  const int rem = m % 64;
-  if (rem > 0 && rem <= 16 && m - rem >= 128 && !gemm_tiles_128x64(m, n)) {
+  if (const int rem = gemm_remainder(m, k, n, BITS)) {
     dispatch<BITS>(x, xs, m - rem, k, packed, scales, bias, n, g, y, ys, s);
     dispatch<BITS>(x + int64_t(m - rem) * xs, xs, rem, k, packed, scales, bias, n, g,
                    y + int64_t(m - rem) * ys, ys, s);
     return;
   }
-  if (gemm_tiles_256(m, n)) {
-    launch_gemm<BITS, 256, 256, 512, 2>(x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
-    return;
+  switch (gemm_tile(m, k, n, BITS)) {
+    case GemmTile::k256:
+      launch_gemm<BITS, 256, 256, 512, 2>(x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
+      break;
+    case GemmTile::k128x256:
+      launch_gemm<BITS, 128, 256, 512, 2>(x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
+      break;
+    case GemmTile::k128:
+      launch_gemm<BITS, 128, 128, EDGERAG_GEMM_THREADS_128, EDGERAG_GEMM_STAGES_128>(
+          x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
+      break;
+    case GemmTile::k128x64:
+      launch_gemm<BITS, 128, 64, EDGERAG_GEMM_THREADS_128x64, EDGERAG_GEMM_STAGES_128x64>(
+          x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
+      break;
+    case GemmTile::k64:
+      launch_gemm<BITS, 64, 64, EDGERAG_GEMM_THREADS_64, EDGERAG_GEMM_STAGES_64>(
+          x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
   }
-  // Tiles: the largest whose grid still covers the 256 CUs.
-  const int64_t t128 = int64_t((n + 127) / 128) * ((m + 127) / 128);
-  if (t128 >= EDGERAG_GEMM_TARGET_WGS)
-    launch_gemm<BITS, 128, 128, EDGERAG_GEMM_THREADS_128, EDGERAG_GEMM_STAGES_128>(
-        x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
-  else if (gemm_tiles_128x64(m, n))
-    launch_gemm<BITS, 128, 64, EDGERAG_GEMM_THREADS_128x64, EDGERAG_GEMM_STAGES_128x64>(
-        x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
-  else
-    launch_gemm<BITS, 64, 64, EDGERAG_GEMM_THREADS_64, EDGERAG_GEMM_STAGES_64>(
-        x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
 }
 
 }  // namespace
@@ -1860,12 +1905,10 @@ bool gemm_rope_shape(int32_t m, int32_t k, int32_t n, int32_t heads, int32_t hea
   if (head_dim != 64 || int64_t(heads) * head_dim != n || m <= EDGERAG_SKINNY_MAX_M ||
       k % kBK != 0)
     return false;
-  const int rem = m % 64;
-  if (rem > 0 && rem <= 16 && m - rem >= 128 && !gemm_tiles_128x64(m, n))
+  if (const int rem = gemm_remainder(m, k, n, 8))
     return gemm_rope_shape(m - rem, k, n, heads, head_dim) &&
            stream_rope_shape(rem, k, n, heads, head_dim);
-  return int64_t((n + 127) / 128) * ((m + 127) / 128) >= EDGERAG_GEMM_TARGET_WGS ||
-         gemm_tiles_128x64(m, n);
+  return gemm_tile(m, k, n, 8) != GemmTile::k64;
 }
 
 template <int MT, bool NORM = false>
@@ -1918,8 +1961,8 @@ void launch_qlinear_rope(const f16* x, int64_t xs, int32_t m, int32_t k, const u
                          const f16* scales, const f16* bias, int32_t n, const EpiArgs& ea,
                          hipStream_t s) {
   if (!stream_rope_shape(m, k, n, ea.n_q_heads + 2 * ea.n_kv_heads, ea.head_dim)) {
-    const int rem = m % 64;
-    if (rem > 0 && rem <= 16 && m - rem >= 128 && !gemm_tiles_128x64(m, n)) {
+    const GemmTile tile = gemm_tile(m, k, n, 8);
+    if (const int rem = gemm_remainder(m, k, n, 8)) {
       launch_qlinear_rope(x, xs, m - rem, k, packed, scales, bias, n, ea, s);
       const int t0 = m - rem;
       EpiArgs er = ea;
@@ -1928,7 +1971,9 @@ void launch_qlinear_rope(const f16* x, int64_t xs, int32_t m, int32_t k, const u
       er.slots += t0;
       er.q_out += int64_t(t0) * ea.q_st;
       launch_qlinear_rope(x + int64_t(t0) * xs, xs, rem, k, packed, scales, bias, n, er, s);
-    } else if (int64_t((n + 127) / 128) * ((m + 127) / 128) >= EDGERAG_GEMM_TARGET_WGS) {
+    } else if (tile == GemmTile::k128x256 || tile == GemmTile::k256) {
+      launch_gemm_rope<256, 512, 2>(x, xs, m, k, packed, scales, bias, n, ea, s);
+    } else if (tile == GemmTile::k128) {
       launch_gemm_rope<128, EDGERAG_GEMM_THREADS_128, EDGERAG_GEMM_STAGES_128>(
           x, xs, m, k, packed, scales, bias, n, ea, s);
     } else {

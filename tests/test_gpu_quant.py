@@ -673,3 +673,32 @@ def test_wide_gemm_tiles_equal_the_narrow_ones(device, bits, k, g, with_bias) ->
     if with_bias:
         ref += bias.float()
     torch.testing.assert_close(got.float(), ref, rtol=1e-2, atol=1e-2 * float(ref.std()))
+
+
+@pytest.mark.parametrize("bits,m,k,n,g,step", [
+    (8, 300, 128, 16300, 128, 100),   # 128x256 tiles, ragged in rows and columns
+    (8, 900, 64, 8100, 64, 100),      # 128x256, the last 4 rows in the same round of tiles
+    (8, 1000, 192, 6100, 64, 100),    # 128x256 with group scales
+    (4, 1500, 256, 4600, 128, 100),   # 128x256, INT4 (432 tiles of 128x128)
+    (8, 520, 128, 6100, 128, 104),    # 128x128 for less than a round, 8 rows past 64-row tiles
+    (8, 1000, 64, 16300, 64, 100),    # 256x256, whose SwiGLU form takes 128x256
+])
+def test_gemm_tiles_of_a_round_equal_the_small_ones(device, bits, m, k, n, g, step) -> None:
+    """Shapes that take 128x256 tiles, 128x128 tiles for less than a round of the CUs, or whose
+    last rows stay in the tiles' launch: every output has the bits of the same rows run ``step``
+    at a time (64x64 to 128x128 tiles; ``step`` leaves no remainder for the streaming kernel),
+    and the SwiGLU form the bits of the projection followed by silu_mul."""
+    gen = torch.Generator(device=device).manual_seed(m + n)
+    packed, scales = kernels.quantize(torch.randn(n, k, generator=gen, device=device) * 0.02, bits, g)
+    bias = torch.randn(n, generator=gen, device=device).half()
+    x = torch.randn(m, k, generator=gen, device=device).half()
+    got = kernels.quant_linear(x, packed, scales, bias, k, n, bits, g, split_k=False)
+    rows = [kernels.quant_linear(x[i : i + step], packed, scales, bias, k, n, bits, g,
+                                 split_k=False) for i in range(0, m, step)]
+    assert torch.equal(got, torch.cat(rows))
+    ref = x.float() @ kernels.dequantize(packed, scales, k, bits, g).float().t() + bias.float()
+    torch.testing.assert_close(got.float(), ref, rtol=1e-2, atol=1e-2 * float(ref.std()))
+    if bits == 8 and g == k:
+        assert kernels.quant_swiglu_fused(m, k, n, bits, g)
+        fused = kernels.quant_linear_swiglu(x, packed, scales, bias, k, n, bits, g)
+        assert torch.equal(fused, kernels.silu_mul(got, n // 2))
