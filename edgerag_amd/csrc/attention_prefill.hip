@@ -20,9 +20,9 @@
 //     once the contraction index is permuted; the A operand is V read transposed out of its
 //     row-major LDS tile (ds_read_b64_tr_b16), four keys of one dim a lane and read.
 //   * fp16 at head_dim 64 rounds p to fp16 (l sums the same rounded p). The other shapes hold p
-//     in 32 bits: p = hi + lo with both halves in the 16-bit type, two MFMAs per step (the
-//     error of hi + lo is 2^-18 of p in bf16, 2^-22 in fp16, against 2^-9 and 2^-11 for the output
-//     rounding), and l sums the fp32 p.
+//     as hi + lo, both halves in the 16-bit type, two MFMAs per step, and l sums the fp32 p: 16
+//     bits of p in bf16 (error 2^-17 of it), 22 in fp16 (2^-22, down to the floor beside
+//     kTopLog2), where the output is rounded to 8 and 11.
 // A wave computes the scores of tile i + 1 while it exponentiates those of tile i, and scales and
 // reduces them while it accumulates P V of tile i: matrix and VALU work that do not depend on each
 // other alternate in the instruction stream. What bounds a tile now is instruction issue: at two
@@ -109,15 +109,27 @@ struct Elem<f16> {
   static __device__ __forceinline__ v4 pack4(float a, float b, float c, float d) {
     return v4{_Float16(a), _Float16(b), _Float16(c), _Float16(d)};
   }
-  // p[0], p[1] as two 16-bit words (round towards zero) and what the rounding left of each.
-  static __device__ __forceinline__ uint32_t head(f2 p) {
+  // The shapes that hold p as hi + lo hold the p of a row's largest score at 2^kTopLog2 and let it
+  // grow to 2^kRaiseLog2. fp16 subnormals end at 2^-24, so hi + lo is off by up to 2^-25 however
+  // small p is: 2^-36 of the largest p here, with at least 22 bits of every p above 2^-14 of it.
+  // (Held at 2^0, the tail behind one dominant key, thousands of keys of 2^-16 to 2^-24 of it, came
+  // out 1% short.)
+  static constexpr float kTopLog2 = 11.f, kRaiseLog2 = 15.f;
+  // p[0], p[1] as two 16-bit words (round towards zero; the one word of fp16 at head_dim 64).
+  static __device__ __forceinline__ uint32_t head_rtz(f2 p) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p[0], p[1]));
+  }
+  // The same rounded to nearest, and what that left of each, rounded to nearest too: rounding
+  // towards zero would take from every key of a long tail what l still counts.
+  static __device__ __forceinline__ uint32_t head(f2 p) {
+    uint32_t w = __builtin_bit_cast(uint32_t, h2{_Float16(p[0]), _Float16(p[1])});
+    asm("" : "+v"(w));  // one packed conversion: else each half is converted again for rest()
+    return w;
   }
   static __device__ __forceinline__ uint32_t rest(f2 p, uint32_t hi) {
     const h2 h = __builtin_bit_cast(h2, hi);
-    return __builtin_bit_cast(
-        uint32_t, __builtin_amdgcn_cvt_pkrtz(__builtin_fmaf(-float(h[0]), 1.f, p[0]),
-                                             __builtin_fmaf(-float(h[1]), 1.f, p[1])));
+    return __builtin_bit_cast(uint32_t, h2{_Float16(__builtin_fmaf(-float(h[0]), 1.f, p[0])),
+                                           _Float16(__builtin_fmaf(-float(h[1]), 1.f, p[1]))});
   }
 };
 template <>
@@ -130,6 +142,7 @@ struct Elem<bf16> {
   static __device__ __forceinline__ v4 pack4(float a, float b, float c, float d) {
     return v4{__bf16(a), __bf16(b), __bf16(c), __bf16(d)};
   }
+  static constexpr float kTopLog2 = 0.f, kRaiseLog2 = kRescaleLog2;  // the exponents of fp32
   static __device__ __forceinline__ uint32_t head(f2 p) {
     return __builtin_bit_cast(uint32_t, b2{__bf16(p[0]), __bf16(p[1])});
   }
@@ -203,6 +216,9 @@ void attn_prefill_mfma_kernel(
   using E = Elem<T>;
   typedef typename E::v8 v8;
   constexpr bool kSplit = !(__is_same(T, f16) && D == 64);  // p as hi + lo (see above)
+  // log2 of the p of a row's largest score, and of the p past which its reference moves.
+  constexpr float kTop = kSplit ? E::kTopLog2 : 0.f;
+  constexpr float kRaise = kSplit ? E::kRaiseLog2 : kRescaleLog2;
   constexpr int kCh = D / 8;                                 // 16-byte chunks of a row
   constexpr int kKpi = kWave / kCh;                          // keys one wave load covers
   constexpr int kLoads = kKeys / kKpi / kWaves;              // wave loads of a tile per wave
@@ -366,16 +382,16 @@ void attn_prefill_mfma_kernel(
   };
 
   // Lazy rescale before the tile whose scores (relative to m) are s with this lane half's
-  // maximum tmax: the reference max m only moves when a score beats it by 2^kRescaleLog2 (before
-  // the first visible score, m is -inf and s is absolute).
+  // maximum tmax: the reference m (the max less kTop) only moves when a p would pass 2^kRaise
+  // (before the first visible score, m is -inf and s is absolute).
   auto rescale = [&](f32x16 (&s)[2], float tmax) {
     tmax = halves_max(tmax);  // the other 16 keys of each 32-key tile
     const bool first = m == -INFINITY;
-    const bool up = first ? tmax != -INFINITY : tmax > kRescaleLog2;
+    const bool up = first ? tmax != -INFINITY : tmax > kRaise;
     if (__any(up)) {
-      const float shift = up ? tmax : 0.f;
+      const float shift = up ? tmax - kTop : 0.f;
       const float alpha = first ? (up ? 0.f : 1.f) : exp2_fast(-shift);
-      if (up) m = first ? tmax : m + tmax;
+      if (up) m = first ? shift : m + shift;
       nm = m == -INFINITY ? 0.f : -m;
       l *= alpha;
 #pragma unroll
@@ -421,12 +437,13 @@ void attn_prefill_mfma_kernel(
       for (int w = c * kPer / 2; w < (c + 1) * kPer / 2; ++w) {
         const int kt = w / 8, i = 2 * (w % 8);
         const f2 p = {exp2_fast(s[kt][i]), exp2_fast(s[kt][i + 1])};
-        hi[w] = E::head(p);
         if constexpr (kSplit) {
+          hi[w] = E::head(p);
           ls[0] += p[0];
           ls[1] += p[1];
           lo[w] = E::rest(p, hi[w]);
         } else {
+          hi[w] = E::head_rtz(p);
           ls[w & 1] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, hi[w]), ones, ls[w & 1], false);
         }
         if constexpr (kNext)

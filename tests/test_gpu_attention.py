@@ -762,3 +762,37 @@ def test_gqa8_workgroup_rows_take_query_vectors_in_passes(device, dtype, n_req) 
     else:  # bf16 keeps 8 bits of mantissa where fp16 keeps 11
         tol = {k_: v_ * 8 for k_, v_ in FP16_TOL.items()}
     torch.testing.assert_close(got.float(), expected, **tol)
+
+
+def _sink_case(L, c, n_q, n_kv, d, dtype, seed, below):
+    """One dominant key whose value row is 0, and every other key ``below`` log2 units (a range)
+    under it: the output is the tail alone, of values large enough for normal fp16 outputs."""
+    g = seeded(seed)
+    kp, vp, tables, qsl, q, bt = _ragged_case([L], [c], n_q, n_kv, d, dtype, seed, poison=False)
+    q = torch.zeros_like(q)
+    q[..., 0] = 8
+    unit = 8 * d**-0.5 * math.log2(math.e)  # log2 units of score per unit of a key's dim 0
+    lo, hi = below
+    kp[..., 0] = (-(lo + (hi - lo) * torch.rand(kp.shape[:-1], generator=g)) / unit).to(dtype)
+    kp[:, tables[0][3], 5, 0] = 0
+    vp = (2.0 ** (lo - 16) * (1 + torch.rand(vp.shape, generator=g))).to(dtype)
+    vp[:, tables[0][3], 5] = 0
+    return kp, vp, tables, qsl, q, bt
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 128), (torch.bfloat16, 64),
+                                     (torch.bfloat16, 128)])
+@pytest.mark.parametrize("L,c", [(4200, 100), (900, 160)])
+def test_tail_behind_a_dominant_key_prefill(device, dtype, d, L, c) -> None:
+    """Probabilities of 2^-16 to 2^-24 of the largest keep their weight in the tiles: against the
+    float64 softmax, with the rounding of the output (2^-9 relative for bf16, 2^-11 for fp16) and
+    nothing for the probabilities."""
+    n_q, n_kv = 4, 2
+    kp, vp, tables, qsl, q, bt = _sink_case(L, c, n_q, n_kv, d, dtype, L + d, (16, 24))
+    got = _run_ragged(device, kp, vp, qsl, [L], bt, q, d**-0.5).double()
+    u = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-11
+    for h in range(n_q):
+        k, v = (op.gather_pool(p.float(), tables[0], L)[h // 2] for p in (kp, vp))
+        ref = oa.attention_f64(q[:, h].float(), k, v, L - c, d**-0.5)
+        assert float(ref.min()) > 2.0**-13  # normal fp16 outputs
+        torch.testing.assert_close(got[:, h], ref, rtol=2 * u, atol=0)
