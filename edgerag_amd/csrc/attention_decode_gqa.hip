@@ -7,10 +7,11 @@
 //   * S^T = K Q^T with v_mfma_f32_16x16x32: K goes from the pool to the A operand in registers
 //     (lane (key, g = lane / 16) loads dims 32 ks + 8 g .. + 7); Q is held as B, the up to 8
 //     vectors in columns 0-7 and again in 8-15.
-//   * softmax in the log2 domain, the reference max raised lazily (when a score beats it by 2^8).
-//   * O^T += V^T P^T with the same MFMA. Probabilities keep 16 + bits: columns 0-7 hold p rounded to
-//     the 16-bit type, columns 8-15 what the rounding left, and the two halves of O add up at the
-//     end, so the split costs no extra MFMA. V goes from the pool straight into a buffer of the
+//   * softmax in the log2 domain, the reference max raised lazily (Elem::kRaiseLog2).
+//   * O^T += V^T P^T with the same MFMA. Columns 0-7 hold p rounded to the 16-bit type, columns 8-15
+//     what the rounding left, and the two halves of O add up at the end, so the split costs no extra
+//     MFMA: 16 bits of p in bf16 (error 2^-17 of it), 22 in fp16 (2^-22, down to the floor beside
+//     kTopLog2), where the output is rounded to 8 and 11; l sums the fp32 p. V goes from the pool straight into a buffer of the
 //     wave in LDS (no staging registers) and is read transposed (ds_read_b64_tr_b16).
 // The next step's K (registers) and V (the other LDS buffer) are in flight while a step is
 // computed; waves do not wait for each other before the merge. Items are run as attn_decode_kernel
@@ -38,7 +39,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kVecs = 8;             // query vectors of an item
 constexpr int kKeys = 32;            // keys per step: two 16-key MFMA tiles
-constexpr float kRescaleLog2 = 8.f;
 constexpr uint32_t kOutOfRange = 0xFFFFF000u;
 
 // Cache policy of the K and V loads: non-temporal, a launch reads each byte once (48 requests,
@@ -69,6 +69,11 @@ struct Elem;
 template <>
 struct Elem<f16> {
   typedef h8 v8;
+  // log2 of the p of a vector's largest score, and of the p past which its reference moves. fp16
+  // subnormals end at 2^-24, so hi + lo is off by up to 2^-25 however small p is: 2^-36 of the
+  // largest p here, with at least 22 bits of every p above 2^-14 of it. (Held at 2^0, keys below
+  // 2^-25 of the largest dropped out of O while l counted them.)
+  static constexpr float kTopLog2 = 11.f, kRaiseLog2 = 15.f;
   static __device__ __forceinline__ f32x4 mfma(v8 a, v8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -85,6 +90,7 @@ struct Elem<f16> {
 template <>
 struct Elem<bf16> {
   typedef b8 v8;
+  static constexpr float kTopLog2 = 0.f, kRaiseLog2 = 8.f;  // the exponents of fp32
   static __device__ __forceinline__ f32x4 mfma(v8 a, v8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
@@ -300,11 +306,11 @@ void attn_decode_gqa_kernel(
       for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[tl][i]);
     tmax = groups_max(tmax);
     const bool first = m == -INFINITY;
-    const bool up = first ? tmax != -INFINITY : tmax > kRescaleLog2;
+    const bool up = first ? tmax != -INFINITY : tmax > E::kRaiseLog2;
     if (__any(up)) {
-      const float shift = up ? tmax : 0.f;
+      const float shift = up ? tmax - E::kTopLog2 : 0.f;
       const float alpha = first ? (up ? 0.f : 1.f) : exp2_fast(-shift);
-      if (up) m = first ? tmax : m + tmax;
+      if (up) m = first ? shift : m + shift;
       nm = m == -INFINITY ? 0.f : -m;
       l *= alpha;
 #pragma unroll

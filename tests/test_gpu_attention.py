@@ -796,3 +796,23 @@ def test_tail_behind_a_dominant_key_prefill(device, dtype, d, L, c) -> None:
         ref = oa.attention_f64(q[:, h].float(), k, v, L - c, d**-0.5)
         assert float(ref.min()) > 2.0**-13  # normal fp16 outputs
         torch.testing.assert_close(got[:, h], ref, rtol=2 * u, atol=0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("L,c,split_rows", [(20000, 1, False), (4200, 2, False), (4200, 2, True)])
+def test_tail_behind_a_dominant_key_grouped_rows(device, dtype, d, L, c, split_rows) -> None:
+    """The same for grouped decode rows, in parts and in KV splits, with probabilities of 2^-24 to
+    2^-28 of the largest, which fp16 holds only above a shifted floor."""
+    n_q, n_kv = 8, 2
+    kp, vp, tables, qsl, q, bt = _sink_case(L, c, n_q, n_kv, d, dtype, L + d, (24, 28))
+    plan, _ = kernels.plan_attention(qsl, np.asarray([L], np.int32), bt, n_q, n_kv, d, BLOCK_SIZE,
+                                     dtype, device, split_rows=split_rows)
+    got = kernels.paged_attention(q.to(device), kp.to(device), vp.to(device), plan,
+                                  d**-0.5).cpu().double()
+    u = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-11
+    for h in range(n_q):
+        k, v = (op.gather_pool(p.float(), tables[0], L)[h // 4] for p in (kp, vp))
+        ref = oa.attention_f64(q[:, h].float(), k, v, L - c, d**-0.5)
+        assert float(ref.min()) > 2.0**-13  # normal fp16 outputs
+        torch.testing.assert_close(got[:, h], ref, rtol=2 * u, atol=0)
