@@ -16,7 +16,9 @@
 // The next step's K (registers) and V (the other LDS buffer) are in flight while a step is
 // computed; waves do not wait for each other before the merge. Items are run as attn_decode_kernel
 // runs them: one wave per KV split, or a workgroup whose waves split the item's keys and merge in
-// LDS. A fused append stores the item's new rows to their slots first and reads them back.
+// LDS. A fused append stores the item's new rows to their slots first and reads them back from the
+// pool, unless a slot is not the row's place in the block table (a padded token's negative slot):
+// the item's new rows then come from the caller's rows, key by key after the others.
 //
 // Bound by the K/V stream at large batches (bf16 32/8 heads of 128, 48 requests of 256-8,192
 // tokens, 870 MB: 213 -> 159 us, 4.1 -> 5.5 TB/s), by the chain of one wave's steps in small ones (one
@@ -196,6 +198,8 @@ void attn_decode_gqa_kernel(
   const uint32_t head_bytes = uint32_t(int64_t(num_blocks) * block_size * D * 2);
   const Slice ks{kpool + head_base * D, head_bytes}, vs{vpool + head_base * D, head_bytes};
 
+  bool detached = false;   // a new row's slot is not its place in the block table
+  const int ke_new = ke;
   if (nk != nullptr && ke > L - c && kb < ke) {
     // The new rows among this wave's keys go to their slots, and are read back below (same wave,
     // after the stores are done).
@@ -207,8 +211,12 @@ void attn_decode_gqa_kernel(
         T* dst = (lane < kCh ? kdst : vdst) + (head_base + slot) * D + lane % kCh * 8;
         store16(dst, load16(src));
       }
+      const int bi = (pos - kb) / block_size;
+      const int blk = __builtin_amdgcn_readlane(my_blk, bi);
+      detached |= blk >= 0 && slot != int64_t(blk) * block_size + (pos - kb - bi * block_size);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (detached) ke = max(kb, L - c);  // the loop takes the keys before the new rows
   }
 
   v8 qop[kKs];
@@ -357,6 +365,32 @@ void attn_decode_gqa_kernel(
   for (int dt = 0; dt < kDt; ++dt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[dt][i] = add_half_row(o[dt][i]);
+  if (detached) {
+    for (int pos = ke; pos < ke_new; ++pos) {
+      if (__builtin_amdgcn_readlane(my_blk, (pos - kb) / block_size) < 0) continue;
+      const int64_t row = int64_t(q0 + pos - (L - c)) * n_st + int64_t(h) * n_sh;
+      float s = 0.f;
+#pragma unroll
+      for (int n = 0; n < kKs; ++n) {
+        const v8 k = *reinterpret_cast<const v8*>(nk + row + 32 * n + 8 * g);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s = __builtin_fmaf(float(qop[n][e]), float(k[e]), s);
+      }
+      s = groups_sum(s) * scale_log2;
+      if (pos > lim) s = -INFINITY;
+      const float top = fmaxf(m, s);
+      const float alpha = m == -INFINITY ? 0.f : exp2_fast(m - top);
+      const float p = s == -INFINITY ? 0.f : exp2_fast(s - top);
+      m = top;
+      l = __builtin_fmaf(l, alpha, p);
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          o[dt][i] = __builtin_fmaf(o[dt][i], alpha,
+                                    p * to_f32<T>(nv[row + 16 * dt + 4 * g + i]));
+    }
+  }
 
   // Register i of O tile dt holds dim 16 dt + 4 g + i of vector `vec`.
   const int64_t row0 = int64_t(part_off) + (int64_t(t - q0) * n_q_heads + hq) * pstride;

@@ -816,3 +816,55 @@ def test_tail_behind_a_dominant_key_grouped_rows(device, dtype, d, L, c, split_r
         ref = oa.attention_f64(q[:, h].float(), k, v, L - c, d**-0.5)
         assert float(ref.min()) > 2.0**-13  # normal fp16 outputs
         torch.testing.assert_close(got[:, h], ref, rtol=2 * u, atol=0)
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.float16, 128),
+                                     (torch.bfloat16, 64), (torch.bfloat16, 128),
+                                     (torch.float32, 64)])
+@pytest.mark.parametrize("n_q,n_kv,c", [(4, 4, 1), (8, 2, 1), (8, 2, 2)])
+@pytest.mark.parametrize("split_rows", [False, True])
+def test_append_fused_attends_rows_whose_slot_is_elsewhere(device, dtype, d, n_q, n_kv, c,
+                                                           split_rows) -> None:
+    """A fused append reads a request's new rows from the caller, whatever their slots: a negative
+    slot (a padded token) writes nothing, one of another block writes there, and attention takes
+    the new row at its position all the same, in one-vector and in grouped rows, at every place
+    in a block, a 32-key step and a context. Against the float64 softmax over the cached keys
+    with the new rows behind them (the tolerances of the grouped rows)."""
+    g = seeded(d + n_q + c)
+    lens = [c, 16, 17, 33, 64, 300, 1201, 2500]
+    q_lens = [c] * len(lens)
+    kp, vp, tables, qsl, q, bt = _ragged_case(lens, q_lens, n_q, n_kv, d, dtype, 77 + d)
+    T = int(qsl[-1])
+    nk, nv = (torch.randn(T, n_kv, d, generator=g).to(dtype) for _ in range(2))
+    spare = [b for b in range(kp.shape[1]) if not any(b in t for t in tables)][0]
+    slots = []
+    for r, L in enumerate(lens):
+        for i in range(c):
+            pos = L - c + i
+            own = tables[r][pos // BLOCK_SIZE] * BLOCK_SIZE + pos % BLOCK_SIZE
+            slots.append([-1, own, spare * BLOCK_SIZE + r][r % 3] if i == 0 else own)
+    slots = np.asarray(slots, np.int32)
+    plan, (slots_d,) = kernels.plan_attention(qsl, np.asarray(lens, np.int32), bt, n_q, n_kv, d,
+                                              BLOCK_SIZE, dtype, device, [slots],
+                                              split_rows=split_rows)
+    assert plan.decode_only
+    kd, vd = kp.to(device), vp.to(device)
+    got = kernels.paged_attention_append(nk.to(device), nv.to(device), slots_d, q.to(device), kd,
+                                         vd, plan, d**-0.5).cpu().double()
+    for pool, new, old in ((kd, nk, kp), (vd, nv, vp)):
+        expect = old.clone()
+        for t, slot in enumerate(slots.tolist()):
+            if slot >= 0:
+                expect[:, slot // BLOCK_SIZE, slot % BLOCK_SIZE] = new[t]
+        assert torch.equal(pool.cpu(), expect)
+    u = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-11
+    tol = FP32_TOL if dtype == torch.float32 else dict(rtol=2 * u, atol=u / 64)
+    for r, L in enumerate(lens):
+        for h in (0, n_q - 1):
+            kv = h // (n_q // n_kv)
+            k, v = (torch.cat([op.gather_pool(p.float(), tables[r], L - c)[kv],
+                               new[qsl[r] : qsl[r + 1], kv].float()])
+                    if L > c else new[qsl[r] : qsl[r + 1], kv].float()
+                    for p, new in ((kp, nk), (vp, nv)))
+            ref = oa.attention_f64(q[qsl[r] : qsl[r + 1], h].float(), k, v, L - c, d**-0.5)
+            torch.testing.assert_close(got[qsl[r] : qsl[r + 1], h], ref, **tol)
