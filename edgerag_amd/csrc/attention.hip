@@ -885,7 +885,7 @@ void dispatch_decode_qr(const Launch& a, int qr, int base, int count, int limit_
   if constexpr (!__is_same(T, float) && (D == 64 || D == 128)) {
     constexpr int32_t kType = __is_same(T, f16) ? EDGERAG_F16 : EDGERAG_BF16;
     if (decode_gqa_supported(a, kType, D, qr, waves)) {
-      launch_decode_gqa(a, kType, D, base, count, limit_word, waves);
+      launch_decode_gqa(a, kType, D, base, count, limit_word, qr, waves);
       return;
     }
   }

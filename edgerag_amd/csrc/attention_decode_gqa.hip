@@ -6,13 +6,14 @@
 // a wave takes 32 keys a step:
 //   * S^T = K Q^T with v_mfma_f32_16x16x32: K goes from the pool to the A operand in registers
 //     (lane (key, g = lane / 16) loads dims 32 ks + 8 g .. + 7); Q is held as B, the up to 8
-//     vectors in columns 0-7 and again in 8-15.
+//     vectors in columns 0-7 and again in 8-15 (bf16, up to 4 vectors: in each 4 columns).
 //   * softmax in the log2 domain, the reference max raised lazily (Elem::kRaiseLog2).
-//   * O^T += V^T P^T with the same MFMA. Columns 0-7 hold p rounded to the 16-bit type, columns 8-15
-//     what the rounding left, and the two halves of O add up at the end, so the split costs no extra
-//     MFMA: 16 bits of p in bf16 (error 2^-17 of it), 22 in fp16 (2^-22, down to the floor beside
-//     kTopLog2), where the output is rounded to 8 and 11; l sums the fp32 p. V goes from the pool straight into a buffer of the
-//     wave in LDS (no staging registers) and is read transposed (ds_read_b64_tr_b16).
+//   * O^T += V^T P^T with the same MFMA. The columns left over hold the rest of each p: fp16 takes
+//     two parts (8 columns each: at least 22 bits down to the floor beside kTopLog2), bf16 three, the
+//     24 bits of fp32: of up to 4 vectors in 4 columns each, of 5 to 8 in 8 columns each and a
+//     second MFMA for the third part. The parts of O add up at the end; l sums the fp32 p. V goes
+//     from the pool straight into a buffer of the wave in LDS (no staging registers) and is read
+//     transposed (ds_read_b64_tr_b16).
 // The next step's K (registers) and V (the other LDS buffer) are in flight while a step is
 // computed; waves do not wait for each other before the merge. Items are run as attn_decode_kernel
 // runs them: one wave per KV split, or a workgroup whose waves split the item's keys and merge in
@@ -33,7 +34,6 @@ using namespace plan;
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef __bf16 b2 __attribute__((ext_vector_type(2)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -96,14 +96,17 @@ struct Elem<bf16> {
   static __device__ __forceinline__ f32x4 mfma(v8 a, v8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
-  static __device__ __forceinline__ uint32_t round2(float a, float b) {
-    return __builtin_bit_cast(uint32_t, b2{__bf16(a), __bf16(b)});
-  }
-  static __device__ __forceinline__ float lo(uint32_t w) { return __uint_as_float(w << 16); }
-  static __device__ __forceinline__ float hi(uint32_t w) {
-    return __uint_as_float(w & 0xFFFF0000u);
-  }
 };
+
+constexpr uint32_t kUpper = 0xFFFF0000u;
+// v less the part of it in the bits of the mask.
+__device__ __forceinline__ float less_upper(float v, uint32_t mask) {
+  return v - __uint_as_float(__float_as_uint(v) & mask);
+}
+// The upper halves of a and b in one word.
+__device__ __forceinline__ uint32_t uppers(float a, float b) {
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302);
+}
 
 // max / sum over the four lanes that differ in lane / 16.
 __device__ __forceinline__ float groups_max(float v) {
@@ -122,10 +125,11 @@ __device__ __forceinline__ float groups_sum(float v) {
                                                   false);
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
-// v plus its value 8 lanes on in the same row of 16 (row_ror:8).
-__device__ __forceinline__ float add_half_row(float v) {
-  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF,
-                                                        false));
+// v of the lane N places on in the same row of 16 (row_shl; 0 past its end).
+template <int N>
+__device__ __forceinline__ float row_ahead(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x100 + N, 0xF, 0xF,
+                                                    true));
 }
 
 // Slot of chunk c of key k in a V buffer row is c ^ v_swizzle(k): 32 lanes of a transposing read
@@ -136,8 +140,9 @@ __device__ __forceinline__ int v_swizzle(int key) {
   return D == 64 ? ((key >> 1) & 3) << 1 : (key & 7) << 1;
 }
 
-// NW: waves per workgroup (1: one wave per item).
-template <typename T, int D, int NW>
+// NW: waves per workgroup (1: one wave per item). VC: columns of a part of the probabilities, 8, or 4
+// for bf16 rows of up to 4 vectors.
+template <typename T, int D, int NW, int VC>
 __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_decode_gqa_kernel(
     const int32_t* __restrict__ plan, int32_t item_base, int32_t limit_word,
@@ -150,6 +155,7 @@ void attn_decode_gqa_kernel(
     int64_t n_st, int64_t n_sh, const int32_t* __restrict__ slots, T* kdst, T* vdst) {
   using E = Elem<T>;
   typedef typename E::v8 v8;
+  constexpr bool kThree = __is_same(T, bf16);  // probabilities in three parts
   constexpr int kKs = D / 32, kDt = D / 16, kCh = D / 8;
   constexpr int kKpi = kWave / kCh;        // keys a V load covers
   constexpr int kVLoads = kKeys / kKpi;
@@ -186,9 +192,12 @@ void attn_decode_gqa_kernel(
   if (lane >= nblk || my_blk >= num_blocks) my_blk = -1;
   const int n_rep = n_q_heads / n_kv_heads;
   const int nvec = qc * n_rep;
-  const int g = lane / 16, col = lane % 16, vec = col % kVecs;
-  const bool low = col >= kVecs;  // this column holds the rounding rests of vector `vec`
+  const int g = lane / 16, col = lane % 16;
+  // This lane's column holds part `part` of the probabilities of vector `vec`.
+  const int part = col / VC, vec = col % VC;
   const bool active = vec < nvec;
+  const uint32_t mask1 = part >= 1 ? kUpper : 0, mask2 = part >= 2 ? kUpper : 0;
+  const uint32_t third_mask = part == 0 ? ~0u : 0;
   const int t = qb + (active ? vec / n_rep : 0);
   const int hq = h * n_rep + (active ? vec % n_rep : 0);
   const int lim = active ? L - c + (t - q0) : -1;
@@ -329,20 +338,34 @@ void attn_decode_gqa_kernel(
         s[1][i] -= shift;
       }
     }
-    u32x4 pw;
+    u32x4 pw, third;  // (third: of 5 to 8 vectors in bf16)
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float p0 = exp2_fast(s[w / 2][2 * (w % 2)]), p1 = exp2_fast(s[w / 2][2 * (w % 2) + 1]);
       l += p0 + p1;
-      const uint32_t head = E::round2(p0, p1);
-      const uint32_t rest = E::round2(p0 - E::lo(head), p1 - E::hi(head));
-      pw[w] = low ? rest : head;
+      if constexpr (kThree) {
+        // The upper half of a float is its first 8 bits in bf16, and what is left is exact.
+        const float a0 = less_upper(p0, mask1), a1 = less_upper(p1, mask1);
+        pw[w] = uppers(less_upper(a0, mask2), less_upper(a1, mask2));
+        if constexpr (VC == 8)
+          third[w] = uppers(less_upper(less_upper(p0, kUpper), kUpper),
+                            less_upper(less_upper(p1, kUpper), kUpper)) & third_mask;
+      } else {
+        const uint32_t head = E::round2(p0, p1);
+        const uint32_t rest = E::round2(p0 - E::lo(head), p1 - E::hi(head));
+        pw[w] = part != 0 ? rest : head;
+      }
     }
     const v8 p = __builtin_bit_cast(v8, pw);
     // This step's V has landed when only the loads of the next step, issued after it, are left.
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kKs + kVLoads) : "memory");
 #pragma unroll
     for (int dt = 0; dt < kDt; ++dt) o[dt] = E::mfma(read_v(sv, dt), p, o[dt]);
+    if constexpr (kThree && VC == 8) {
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt)
+        o[dt] = E::mfma(read_v(sv, dt), __builtin_bit_cast(v8, third), o[dt]);
+    }
   };
 
   char* const buf0 = sv0 + wave * kBuf;
@@ -364,7 +387,10 @@ void attn_decode_gqa_kernel(
 #pragma unroll
   for (int dt = 0; dt < kDt; ++dt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[dt][i] = add_half_row(o[dt][i]);
+    for (int i = 0; i < 4; ++i) {
+      const float v = o[dt][i];
+      o[dt][i] += VC == 4 ? row_ahead<4>(v) + row_ahead<8>(v) : row_ahead<8>(v);
+    }
   if (detached) {
     for (int pos = ke; pos < ke_new; ++pos) {
       if (__builtin_amdgcn_readlane(my_blk, (pos - kb) / block_size) < 0) continue;
@@ -395,7 +421,7 @@ void attn_decode_gqa_kernel(
   // Register i of O tile dt holds dim 16 dt + 4 g + i of vector `vec`.
   const int64_t row0 = int64_t(part_off) + (int64_t(t - q0) * n_q_heads + hq) * pstride;
   if constexpr (NW == 1) {
-    if (!active || low) return;
+    if (!active || part != 0) return;
     if (nsplit == 1) {
       const float inv = 1.f / fmaxf(l, 1.17549435e-38f);
       T* op = out + int64_t(t) * o_st + int64_t(hq) * o_sh;
@@ -413,7 +439,7 @@ void attn_decode_gqa_kernel(
   } else {
     // The waves' (m, l, O) meet in their own V buffers; the workgroup merges and writes.
     float* acc0 = reinterpret_cast<float*>(buf0);
-    if (active && !low) {
+    if (active && part == 0) {
 #pragma unroll
       for (int dt = 0; dt < kDt; ++dt)
         *reinterpret_cast<f32x4*>(acc0 + vec * D + 16 * dt + 4 * g) = o[dt];
@@ -451,9 +477,9 @@ void attn_decode_gqa_kernel(
   }
 }
 
-template <typename T, int D, int NW>
-void launch(const AttnLaunch& a, int base, int count, int limit_word) {
-  hipLaunchKernelGGL((attn_decode_gqa_kernel<T, D, NW>), dim3(count), dim3(NW * kWave), 0, a.s,
+template <typename T, int D, int NW, int VC>
+void launch_kernel(const AttnLaunch& a, int base, int count, int limit_word) {
+  hipLaunchKernelGGL((attn_decode_gqa_kernel<T, D, NW, VC>), dim3(count), dim3(NW * kWave), 0, a.s,
                      a.plan, base, limit_word, a.qsl, a.ctx, a.bt, a.bt_stride, a.nb, a.bs,
                      static_cast<const T*>(a.q), a.q_st, a.q_sh, static_cast<const T*>(a.kp),
                      static_cast<const T*>(a.vp), a.hq, a.hkv, a.scale_log2,
@@ -463,20 +489,28 @@ void launch(const AttnLaunch& a, int base, int count, int limit_word) {
                      static_cast<T*>(const_cast<void*>(a.vp)));
 }
 
+template <typename T, int D, int NW>
+void launch(const AttnLaunch& a, int base, int count, int limit_word, int vecs) {
+  if (__is_same(T, bf16) && vecs <= 4)
+    launch_kernel<T, D, NW, __is_same(T, bf16) ? 4 : 8>(a, base, count, limit_word);
+  else
+    launch_kernel<T, D, NW, 8>(a, base, count, limit_word);
+}
+
 // Waves of a workgroup row this kernel is built for: those the planner gives rows of the head_dim.
 bool row_waves_built(int32_t head_dim, int waves) {
   return waves == 0 || (head_dim == 64 ? waves == 8 || waves == 16 : waves == kGqaWaves);
 }
 
 template <typename T, int D>
-void launch_waves(const AttnLaunch& a, int base, int count, int limit_word, int waves) {
+void launch_waves(const AttnLaunch& a, int base, int count, int limit_word, int vecs, int waves) {
   if (waves == 0) {
-    launch<T, D, 1>(a, base, count, limit_word);
+    launch<T, D, 1>(a, base, count, limit_word, vecs);
   } else if constexpr (D == 64) {
-    if (waves == 8) launch<T, D, 8>(a, base, count, limit_word);
-    else launch<T, D, 16>(a, base, count, limit_word);
+    if (waves == 8) launch<T, D, 8>(a, base, count, limit_word, vecs);
+    else launch<T, D, 16>(a, base, count, limit_word, vecs);
   } else {
-    launch<T, D, kGqaWaves>(a, base, count, limit_word);
+    launch<T, D, kGqaWaves>(a, base, count, limit_word, vecs);
   }
 }
 
@@ -494,14 +528,14 @@ bool decode_gqa_supported(const AttnLaunch& a, int32_t dtype, int32_t head_dim, 
 }
 
 void launch_decode_gqa(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int base, int count,
-                       int limit_word, int waves) {
+                       int limit_word, int vecs, int waves) {
   const bool half = dtype == EDGERAG_F16;
   if (head_dim == 64) {
-    if (half) launch_waves<f16, 64>(a, base, count, limit_word, waves);
-    else launch_waves<bf16, 64>(a, base, count, limit_word, waves);
+    if (half) launch_waves<f16, 64>(a, base, count, limit_word, vecs, waves);
+    else launch_waves<bf16, 64>(a, base, count, limit_word, vecs, waves);
   } else {
-    if (half) launch_waves<f16, 128>(a, base, count, limit_word, waves);
-    else launch_waves<bf16, 128>(a, base, count, limit_word, waves);
+    if (half) launch_waves<f16, 128>(a, base, count, limit_word, vecs, waves);
+    else launch_waves<bf16, 128>(a, base, count, limit_word, vecs, waves);
   }
 }
 

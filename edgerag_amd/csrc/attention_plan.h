@@ -103,7 +103,7 @@ bool decode_gqa_shape(int32_t dtype, int32_t head_dim, int vecs, int32_t block_s
 bool decode_gqa_supported(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int vecs,
                           int waves);
 void launch_decode_gqa(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int base, int count,
-                       int limit_word, int waves);
+                       int limit_word, int vecs, int waves);
 // Prefill tiles in fp32 (attention_prefill_f32.hip), head_dim 64 and 128: 16 or 32 virtual rows.
 void launch_prefill_f32(const AttnLaunch& a, int32_t head_dim, int rows, int item_base, int count);
 bool prefill_f32_supported(int32_t num_blocks, int32_t block_size, int32_t head_dim);

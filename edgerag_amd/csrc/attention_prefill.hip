@@ -21,7 +21,7 @@
 //     row-major LDS tile (ds_read_b64_tr_b16), four keys of one dim a lane and read.
 //   * fp16 at head_dim 64 rounds p to fp16 (l sums the same rounded p). The other shapes hold p
 //     as hi + lo, both halves in the 16-bit type, two MFMAs per step, and l sums the fp32 p: 16
-//     bits of p in bf16 (error 2^-17 of it), 22 in fp16 (2^-22, down to the floor beside
+//     bits of p in bf16 (error 2^-16 of it), 22 in fp16 (2^-22, down to the floor beside
 //     kTopLog2), where the output is rounded to 8 and 11.
 // A wave computes the scores of tile i + 1 while it exponentiates those of tile i, and scales and
 // reduces them while it accumulates P V of tile i: matrix and VALU work that do not depend on each

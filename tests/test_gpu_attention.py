@@ -401,8 +401,8 @@ def test_wide_prefill_tile_edges(device, dtype, d, n_q, n_kv) -> None:
     """The tiles that hold p in 32 bits (the fp32 ones too): one token past the row limit, one short of and past a
     128-row tile, chunks below, at and past a 64-key tile, odd prefixes and a split context, all
     in one batch whose unwritten pool rows are NaN, against the float64 softmax. The error is the
-    rounding of the output (2^-9 relative for bf16, 2^-11 for fp16) plus that of hi + lo
-    (2^-17, 2^-22)."""
+    rounding of the output (2^-8 relative for bf16, 2^-11 for fp16) plus that of hi + lo
+    (2^-16, 2^-22)."""
     rep = n_q // n_kv
     chunks = [8 // rep + 1, 64, 65, 128 // rep - 1, 128 // rep + 1, 200]
     lens = [c + p for c, p in zip(chunks, [0, 0, 13, 64, 250, 1900])]
@@ -868,3 +868,33 @@ def test_append_fused_attends_rows_whose_slot_is_elsewhere(device, dtype, d, n_q
                     for p, new in ((kp, nk), (vp, nv)))
             ref = oa.attention_f64(q[qsl[r] : qsl[r + 1], h].float(), k, v, L - c, d**-0.5)
             torch.testing.assert_close(got[qsl[r] : qsl[r + 1], h], ref, **tol)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n_q,n_kv,reqs", [(8, 2, 40), (10, 2, 40), (16, 2, 40), (8, 2, 400)])
+def test_grouped_rows_hold_probabilities_in_fp32_bf16(device, d, n_q, n_kv, reqs) -> None:
+    """bf16 rows whose output is the difference of two nearly equal probabilities: contexts of two
+    keys whose scores differ by about 2^-11 and whose values are opposite, and a third, of value 0,
+    above them (so that neither probability is a short number). The output keeps its 8
+    bits only if each probability has the 24 of fp32 (two bf16 parts, 16 bits, were off by up to
+    2%): the scores' and exponentials' fp32 rounding is 2^-22 of the probabilities, 2^-9 of
+    their difference, beside the 2^-8 of the output's rounding. Up to 4 vectors and more, in
+    workgroup rows and (400 requests) KV splits."""
+    g = seeded(d + n_q)
+    lens = [3] * reqs
+    kp, vp, tables, qsl, q, bt = _ragged_case(lens, [1] * reqs, n_q, n_kv, d, torch.bfloat16, 5)
+    q = torch.zeros_like(q)
+    q[..., 0], q[..., 1] = 1, 2.0**-8 if d == 64 else 2.0**-7
+    kp = torch.zeros_like(kp)
+    kp[:, :, 0, 0] = torch.randn(kp.shape[:2], generator=g).to(kp.dtype)
+    kp[:, :, 1, 0] = kp[:, :, 0, 0]
+    kp[:, :, 2, 0] = kp[:, :, 0, 0] + (1 + 3 * torch.rand(kp.shape[:2], generator=g)).to(kp.dtype)
+    kp[:, :, 0, 1] = (0.5 + torch.rand(kp.shape[:2], generator=g)).to(kp.dtype)
+    vp[:, :, 0] = (1 + torch.rand(vp[:, :, 0].shape, generator=g)).to(vp.dtype)
+    vp[:, :, 1], vp[:, :, 2] = -vp[:, :, 0], 0
+    got = _run_ragged(device, kp, vp, qsl, lens, bt, q, d**-0.5).double()
+    for r in range(0, reqs, 7):
+        for h in range(n_q):
+            k, v = (op.gather_pool(p.float(), tables[r], 3)[h // (n_q // n_kv)] for p in (kp, vp))
+            ref = oa.attention_f64(q[r : r + 1, h].float(), k, v, 2, d**-0.5)
+            torch.testing.assert_close(got[r : r + 1, h], ref, rtol=2.0**-8 + 2.0**-9, atol=0)
