@@ -229,6 +229,10 @@ void attn_prefill_mfma_kernel(
   __shared__ __align__(16) char sk0[kKeys * D * 2], sk1[kKeys * D * 2];
   __shared__ __align__(16) char sv0[kKeys * D * 2], sv1[kKeys * D * 2];
   __shared__ uint32_t sblk[kMaxTileBlocks];  // byte offset of each block in the head's slice
+  __shared__ struct {
+    const T* q;
+    int64_t st, sh;
+  } sq;  // q again, for the rare sum after the last tile: no register holds it across the loop
 
   if (EDGERAG_TILE_PRIO > 0) __builtin_amdgcn_s_setprio(EDGERAG_TILE_PRIO);
   const int32_t* it = plan + plan[H_ITEM_OFF] + int64_t(item_base + blockIdx.x) * kItemWords;
@@ -266,6 +270,11 @@ void attn_prefill_mfma_kernel(
   // Whether any of them is invalid (never in a well-formed table) decides once per item whether
   // tiles check for invalid keys.
   int any_bad = 0;
+  if (tid == 0) {
+    sq.q = q;
+    sq.st = q_st;
+    sq.sh = q_sh;
+  }
   {
     const int nblk = min(((ke - 1) >> bs_shift) - geo.blk0 + 1, kMaxTileBlocks);
     for (int i = tid; i < nblk; i += kThreads) {
@@ -565,6 +574,53 @@ void attn_prefill_mfma_kernel(
   // No load may still be on its way into this workgroup's LDS when the workgroup ends.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   l = halves_sum(l);
+
+  // A key that a row does not see has p = 0, and 0 times a NaN or infinite V is NaN: a later token's
+  // V must not reach the rows before it. Where one did, the rows are summed again key by key.
+  float any_odd = 0.f;
+#pragma unroll
+  for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) any_odd = __builtin_fmaf(o[dt][i], 0.f, any_odd);
+  if (__any(active && any_odd != 0.f)) {
+    auto row_of = [&](int pos) {  // byte offset of key pos in the head's slice
+      return __builtin_elementwise_add_sat(sblk[(pos >> bs_shift) - geo.blk0],
+                                           uint32_t(pos & geo.bs_mask) * uint32_t(D * 2));
+    };
+    auto finite = [](T v) { return __builtin_fabsf(to_f32<T>(v)) < INFINITY; };
+    bool hidden = false;  // a non-finite V among the keys that some row of the wave does not see
+    for (int pos = max(kb, wave_min_lim + 1) + lane / kCh; pos < ke; pos += kKpi) {
+      const uint32_t off = row_of(pos);
+      const T* v = reinterpret_cast<const T*>(static_cast<const char*>(vrs.base) + off);
+      for (int e = 0; e < 8; ++e) hidden |= off < vrs.bytes && !finite(v[8 * (lane % kCh) + e]);
+    }
+    if (__any(hidden)) {
+      const T* qp = sq.q + int64_t(t) * sq.st + int64_t(hq) * sq.sh;
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt) o[dt] = f32x16{};
+      for (int pos = kb; pos < ke; ++pos) {
+        const uint32_t off = row_of(pos);
+        if (off >= vrs.bytes) continue;
+        const T* k = reinterpret_cast<const T*>(static_cast<const char*>(krs.base) + off);
+        const T* v = reinterpret_cast<const T*>(static_cast<const char*>(vrs.base) + off);
+        float s = 0.f;
+        for (int ks = 0; ks < kKs; ++ks)
+#pragma unroll
+          for (int e = 16 * ks + 8 * g; e < 16 * ks + 8 * g + 8; ++e)
+            s = __builtin_fmaf(to_f32<T>(qp[e]), to_f32<T>(k[e]), s);
+        float p = exp2_fast(__builtin_fmaf(halves_sum(s), scale_log2, nm));
+        if constexpr (!kSplit)
+          p = float(__builtin_bit_cast(h2, E::head_rtz(f2{p, 0.f}))[0]);
+        if (pos > lim) continue;
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            o[dt][i] = __builtin_fmaf(
+                p, to_f32<T>(v[32 * dt + (i & 3) + 8 * (i >> 2) + 4 * g]), o[dt][i]);
+      }
+    }
+  }
 
   if (!active) return;
   // O^T register i of dim tile dt holds dim 32dt + (i%4) + 8(i/4) + 4g of this lane's query.

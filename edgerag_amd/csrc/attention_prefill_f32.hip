@@ -288,6 +288,33 @@ __global__ __launch_bounds__(kThreads) void attn_prefill_f32_kernel(
       for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(wgt, v[e], acc[e]);
     }
     const int t = qb + rho / n_rep, hq = h * n_rep + rho % n_rep;
+    // A key that a row does not see has p = 0, and 0 times a NaN or infinite V is NaN: a later
+    // token's V must not reach the rows before it. Where one did, the row's keys are summed again.
+    const float odd = (acc[0] + acc[1] + acc[2] + acc[3]) * 0.f;
+    if (odd != 0.f) {
+      const int seen = min(ke, L - c + (t - q0) + 1);
+      bool hidden = false;
+      for (int pos = max(kb, seen); pos < ke; ++pos) {
+        const f32x4 v = load_slice(vs, __builtin_elementwise_add_sat(row_offset(pos), uint32_t(4 * d)));
+        for (int e = 0; e < 4; ++e) hidden |= !(__builtin_fabsf(v[e]) < INFINITY);
+      }
+      if (hidden) {
+        const float* qp = q + int64_t(t) * q_st + int64_t(hq) * q_sh;
+        acc = f32x4{};
+        for (int pos = kb; pos < seen; ++pos) {
+          const uint32_t off = row_offset(pos);
+          if (off >= head_bytes) continue;
+          float dot = 0.f;
+          for (int e = 0; e < D; e += 4) {
+            const f32x4 k = load_slice(ks, off + uint32_t(4 * e));
+            for (int x = 0; x < 4; ++x) dot = __builtin_fmaf(qp[e + x] * scale_log2, k[x], dot);
+          }
+          const float p = exp2_fast(dot - mx);
+          const f32x4 v = load_slice(vs, off + uint32_t(4 * d));
+          for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(p, v[e], acc[e]);
+        }
+      }
+    }
     if (nsplit == 1) {
       const float inv = 1.f / fmaxf(lsum, 1.17549435e-38f);
       float* dst = out + int64_t(t) * o_st + int64_t(hq) * o_sh + d;

@@ -898,3 +898,38 @@ def test_grouped_rows_hold_probabilities_in_fp32_bf16(device, d, n_q, n_kv, reqs
             k, v = (op.gather_pool(p.float(), tables[r], 3)[h // (n_q // n_kv)] for p in (kp, vp))
             ref = oa.attention_f64(q[r : r + 1, h].float(), k, v, 2, d**-0.5)
             torch.testing.assert_close(got[r : r + 1, h], ref, rtol=2.0**-8 + 2.0**-9, atol=0)
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.bfloat16, 64),
+                                     (torch.float16, 128), (torch.bfloat16, 128),
+                                     (torch.float32, 64), (torch.float32, 128)])
+@pytest.mark.parametrize("n_q,n_kv,reqs", [(4, 4, 1), (6, 2, 1), (4, 4, 40)])
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+def test_non_finite_values_of_later_tokens_stay_hidden(device, dtype, d, n_q, n_kv, reqs,
+                                                       bad) -> None:
+    """A NaN or infinite value row of a slice's own token reaches that token and those after it and
+    no other, whatever tile the rows share: the rows before it match the float64 softmax (which
+    does not see it), those after show it in its dims. Slices behind prefixes with a bad row in
+    their middle or in their last token, split contexts, and (40 requests) 32-row fp32 tiles."""
+    chunks = ([150, 70, 300] if reqs == 1 else [33]) * reqs
+    past = ([0, 1000, 2500] if reqs == 1 else [40]) * reqs
+    at = ([100, 69, 130] if reqs == 1 else [20]) * reqs  # the token whose value row is bad
+    lens = [c + p for c, p in zip(chunks, past)]
+    kp, vp, tables, qsl, q, bt = _ragged_case(lens, chunks, n_q, n_kv, d, dtype, 9 + d)
+    for r, (p, a) in enumerate(zip(past, at)):
+        vp[:, tables[r][(p + a) // BLOCK_SIZE], (p + a) % BLOCK_SIZE, 5 : d // 2] = bad
+    got = _run_ragged(device, kp, vp, qsl, lens, bt, q, d**-0.5).double()
+    u = {torch.bfloat16: 2.0**-9, torch.float16: 2.0**-11}.get(dtype)
+    tol = FP32_TOL if u is None else FP16_TOL if (dtype, d) == (torch.float16, 64) else dict(
+        rtol=2 * u, atol=u / 64)
+    for r in range(0, len(lens), 13 if reqs > 1 else 1):
+        for h in (0, n_q - 1):
+            k, v = (op.gather_pool(p.float(), tables[r], lens[r])[h // (n_q // n_kv)]
+                    for p in (kp, vp))
+            v = v.clone()
+            v[past[r] + at[r]] = 0  # not seen by the rows compared
+            out, a = got[qsl[r] : qsl[r + 1], h], at[r]
+            ref = oa.attention_f64(q[qsl[r] : qsl[r + 1], h].float(), k, v, past[r], d**-0.5)
+            torch.testing.assert_close(out[:a], ref[:a], **tol)
+            assert not out[a:, 5 : d // 2].isfinite().any()
+            assert out[a:, : 5].isfinite().all() and out[a:, d // 2 :].isfinite().all()
