@@ -998,8 +998,12 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
                 max_blocks_per_seq);
 
   const int n_rep = n_q_heads / n_kv_heads;
-  // Prefill tiles on MFMA: 128 virtual rows (token x head-in-group).
-  const bool mfma_tiles = prefill_tile_shape(dtype, head_dim) && n_rep <= kMfmaTileRows;
+  // Prefill tiles on MFMA: 128 virtual rows (token x head-in-group), for the block sizes its kernel
+  // takes. The others run on the row kernel, one wave an item, in items of kQTile tokens: 512 tokens
+  // at 2,048 keys in blocks of 48, bf16, items of 128 rows / of kQTile tokens: 32/32 heads of 64
+  // 2,114 / 515 us, 32/8 of 128 4,075 / 2,184.
+  const bool mfma_tiles = prefill_tile_shape(dtype, head_dim) && n_rep <= kMfmaTileRows &&
+                          prefill_tiles_supported(1, block_size, head_dim);
   // In fp32 on 16 or 32 virtual rows: 16 for batches of few tiles (short prompts, where the chain
   // of one workgroup's chunks is the time), else 32, which read K and V half as often.
   int tile_kind = mfma_tiles ? 1 : 0;

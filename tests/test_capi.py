@@ -453,6 +453,22 @@ def test_wide_tile_partials_fit_the_static_scratch(n_q, n_kv) -> None:
             assert all(int(reqs[r][1]) % 64 == 0 for r in range(n))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n_q,n_kv", [(32, 32), (32, 8)])
+def test_prefill_items_fit_the_kernel_that_takes_the_blocks(dtype, d, n_q, n_kv) -> None:
+    """Prefill items hold 128 rows (token x head of the group) where the MFMA tiles take the block
+    size, and 16 tokens where it is below 4 or no power of two: the row kernel runs those with one
+    wave an item."""
+    for bs in (1, 2, 3, 4, 8, 16, 24, 48, 64):
+        qsl, ctx = _mixed([(512, 1536)], [])
+        plan, _ = kernels.make_plan_host(qsl, ctx, n_q, n_kv, d, bs, 2048, dtype)
+        mfma = bs >= 4 and bs & (bs - 1) == 0
+        items, _reqs = decode_plan(plan)
+        assert int(plan[18]) == (1 if mfma else 0), bs
+        assert int(items[:, 3].max()) == (128 * n_kv // n_q if mfma else 16), bs
+
+
 @pytest.mark.parametrize("slices,decodes,force,overlap", [
     # config 3: 384 tiles (every CU at one workgroup) beside 24 decodes reading 707 MB
     ([(512, 0), (512, 3584), (512, 6656)], "cfg3", False, 1),
