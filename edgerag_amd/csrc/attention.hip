@@ -880,8 +880,8 @@ void dispatch_decode_qr(const Launch& a, int qr, int base, int count, int limit_
                         int waves) {
   constexpr int U = D >= 256 ? 2 : kDecodeU;
   // Two or more query vectors a row: the matrix cores (attention_decode_gqa.hip), where the VALU
-  // kernel is bound by its arithmetic (bf16 32/8 heads of 128, 48 requests 216 -> 159 us; two vectors,
-  // fp16 16/8 of 128, 32 requests, 77.6 -> 74.7).
+  // kernel is bound by its arithmetic (bf16 32/8 heads of 128, 48 requests of 4,000 tokens 154.8 ->
+  // 141.5 us, of 32/8 heads of 64 88.8 -> 68.1); decode_gqa_supported says which rows of two.
   if constexpr (!__is_same(T, float) && (D == 64 || D == 128)) {
     constexpr int32_t kType = __is_same(T, f16) ? EDGERAG_F16 : EDGERAG_BF16;
     if (decode_gqa_supported(a, kType, D, qr, waves)) {

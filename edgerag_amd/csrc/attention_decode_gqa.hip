@@ -521,8 +521,17 @@ bool decode_gqa_shape(int32_t dtype, int32_t head_dim, int vecs, int32_t block_s
          vecs >= 2 && vecs <= kVecs && block_size % 16 == 0;
 }
 
+// Rows of two vectors as KV splits, one wave an item in batches large enough to be bound by the
+// stream, stay on attn_decode_kernel, whose loads run further ahead, but for bf16 at head_dim 64,
+// whose fp32 query registers bind it there. Here / there, us: fp16 16/8 heads of 128, 32 requests of
+// 256-7,472 tokens 100.7 / 95.4, 48 of 4,000 133.1 / 128.8; bf16 32/16 of 128, 48 of 4,000 259.0 /
+// 249.3; fp16 64/32 of 64, 48 of 4,000 260.9 / 247.8, 32/16 of 64, 32 of 256-7,472 96.2 / 95.1; bf16
+// 32/16 of 64 96.3 / 106.9. (fp16 32/16 of 64, 32 of 2,000: 46.4 / 48.6, the one the other way.)
+// Workgroup rows are bound by a wave's chain: fp16 32/16 of 64, 8 requests of 256-3,000 16.1 / 22.5.
+// Three vectors: fp16 24/8 of 128, 64 of 256-4,096 105.4 / 109.7.
 bool decode_gqa_supported(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int vecs,
                           int waves) {
+  if (vecs == 2 && waves == 0 && !(dtype == EDGERAG_BF16 && head_dim == 64)) return false;
   return decode_gqa_shape(dtype, head_dim, vecs, a.bs) && row_waves_built(head_dim, waves) &&
          int64_t(a.nb) * a.bs * head_dim * 2 < int64_t(kOutOfRange);
 }

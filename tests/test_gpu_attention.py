@@ -933,3 +933,20 @@ def test_non_finite_values_of_later_tokens_stay_hidden(device, dtype, d, n_q, n_
             torch.testing.assert_close(out[:a], ref[:a], **tol)
             assert not out[a:, 5 : d // 2].isfinite().any()
             assert out[a:, : 5].isfinite().all() and out[a:, d // 2 :].isfinite().all()
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 64), (torch.float16, 128),
+                                     (torch.bfloat16, 128)])
+def test_one_request_of_two_tokens_leaves_the_other_rows_as_they_are(device, dtype, d) -> None:
+    """Multi-head decode rows in KV splits: one request that brings two tokens makes two-vector rows
+    of its own and does not move the others to another kernel (which is slower for them): their
+    outputs keep their bits."""
+    lens = [700, 33, 1500, 128, 900, 64]
+    kp, vp, tables, qsl, q, bt = _ragged_case(lens, [1] * 5 + [2], 4, 4, d, dtype, d)
+    outs = []
+    for n in (5, 6):
+        plan, _ = kernels.plan_attention(qsl[: n + 1], np.asarray(lens[:n], np.int32), bt[:n], 4, 4,
+                                         d, BLOCK_SIZE, dtype, device, split_rows=True)
+        outs.append(kernels.paged_attention(q[: int(qsl[n])].to(device), kp.to(device),
+                                            vp.to(device), plan, d**-0.5))
+    assert torch.equal(outs[0], outs[1][:5])
