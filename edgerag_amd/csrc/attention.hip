@@ -877,14 +877,14 @@ void launch_rows(const Launch& a, int base, int count, int limit_word) {
 
 template <typename T, int D>
 void dispatch_decode_qr(const Launch& a, int qr, int base, int count, int limit_word,
-                        int waves) {
+                        int waves, bool tiles = false) {
   constexpr int U = D >= 256 ? 2 : kDecodeU;
   // Two or more query vectors a row: the matrix cores (attention_decode_gqa.hip), where the VALU
   // kernel is bound by its arithmetic (bf16 32/8 heads of 128, 48 requests of 4,000 tokens 154.8 ->
   // 141.5 us, of 32/8 heads of 64 88.8 -> 68.1); decode_gqa_supported says which rows of two.
   if constexpr (!__is_same(T, float) && (D == 64 || D == 128)) {
     constexpr int32_t kType = __is_same(T, f16) ? EDGERAG_F16 : EDGERAG_BF16;
-    if (decode_gqa_supported(a, kType, D, qr, waves)) {
+    if (decode_gqa_supported(a, kType, D, qr, waves, tiles)) {
       launch_decode_gqa(a, kType, D, base, count, limit_word, qr, waves);
       return;
     }
@@ -946,7 +946,7 @@ int run_items(const Launch& a, const int32_t* ph, int parts) {
   const bool fast = a.bs % C::TPW == 0 && ph[H_MAX_SPLIT_BLOCKS] <= kMaxSplitBlocks;
   if ((parts & EDGERAG_ATTN_ROWS) && n_row > 0) {
     if (fast)
-      dispatch_decode_qr<T, D>(a, qr, 0, n_row, H_N_ROW_ITEMS, ph[H_ROW_WAVES]);
+      dispatch_decode_qr<T, D>(a, qr, 0, n_row, H_N_ROW_ITEMS, ph[H_ROW_WAVES], n_items > n_row);
     else  // (workgroup-split rows are only planned for the fast kernel)
       dispatch_rows_qr<T, D>(a, qr, 0, n_row, H_N_ROW_ITEMS);
   }

@@ -527,11 +527,14 @@ bool decode_gqa_shape(int32_t dtype, int32_t head_dim, int vecs, int32_t block_s
 // 256-7,472 tokens 100.7 / 95.4, 48 of 4,000 133.1 / 128.8; bf16 32/16 of 128, 48 of 4,000 259.0 /
 // 249.3; fp16 64/32 of 64, 48 of 4,000 260.9 / 247.8, 32/16 of 64, 32 of 256-7,472 96.2 / 95.1; bf16
 // 32/16 of 64 96.3 / 106.9. (fp16 32/16 of 64, 32 of 2,000: 46.4 / 48.6, the one the other way.)
+// After or beside prefill tiles (tiles) the arithmetic of attn_decode_kernel takes longer than alone:
+// head_dim 128 then stays here (two 512-token slices and 30 decodes of 4,096, 32/16 heads of 128,
+// bf16 231 / 274, fp16 232 / 240; four slices and 40 of 512-7,472, 16/8 188 / 227, 189 / 201).
 // Workgroup rows are bound by a wave's chain: fp16 32/16 of 64, 8 requests of 256-3,000 16.1 / 22.5.
 // Three vectors: fp16 24/8 of 128, 64 of 256-4,096 105.4 / 109.7.
 bool decode_gqa_supported(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int vecs,
-                          int waves) {
-  if (vecs == 2 && waves == 0 && !(dtype == EDGERAG_BF16 && head_dim == 64)) return false;
+                          int waves, bool tiles) {
+  if (vecs == 2 && waves == 0 && (head_dim == 128 ? !tiles : dtype == EDGERAG_F16)) return false;
   return decode_gqa_shape(dtype, head_dim, vecs, a.bs) && row_waves_built(head_dim, waves) &&
          int64_t(a.nb) * a.bs * head_dim * 2 < int64_t(kOutOfRange);
 }

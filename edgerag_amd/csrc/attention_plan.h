@@ -98,10 +98,11 @@ bool prefill_tiles_supported(int32_t num_blocks, int32_t block_size, int32_t hea
 constexpr int kGqaWaves = 4;  // waves of a workgroup row of the GQA kernel at head_dim 128
 // Decode rows with 2 to 8 query vectors on MFMA (attention_decode_gqa.hip): fp16 and bf16, head_dim
 // 64 and 128, one wave per item or workgroup rows.
-// Whether the kernel is built for the shape, and whether it takes this launch.
+// Whether the kernel is built for the shape, and whether it takes this launch (tiles: of a plan that
+// holds prefill tiles as well).
 bool decode_gqa_shape(int32_t dtype, int32_t head_dim, int vecs, int32_t block_size);
 bool decode_gqa_supported(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int vecs,
-                          int waves);
+                          int waves, bool tiles);
 void launch_decode_gqa(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int base, int count,
                        int limit_word, int vecs, int waves);
 // Prefill tiles in fp32 (attention_prefill_f32.hip), head_dim 64 and 128: 16 or 32 virtual rows.
