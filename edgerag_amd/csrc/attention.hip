@@ -925,11 +925,16 @@ template <typename T, int D>
 int run_items(const Launch& a, const int32_t* ph, int parts) {
   using C = RowCfg<T, D>;
   const int n_items = ph[H_N_ITEMS], n_row = ph[H_N_ROW_ITEMS];
+  const int qr = std::min(8, pow2_at_least(std::max(1, ph[H_MAX_ROW_VECS])));
+  const bool fast = a.bs % C::TPW == 0 && ph[H_MAX_SPLIT_BLOCKS] <= kMaxSplitBlocks;
   if ((parts & EDGERAG_ATTN_TILES) && n_items > n_row) {
     if constexpr (!__is_same(T, float) && (D == 64 || D == 128)) {
       if (ph[H_TILE_KIND] == 1 && prefill_tiles_supported(a.nb, a.bs, D)) {
+        const bool gqa =
+            fast && decode_gqa_supported(a, ph[H_DTYPE], D, qr, ph[H_ROW_WAVES], true);
         launch_prefill_tiles(a, ph[H_DTYPE], D, n_row, n_items - n_row,
-                             (parts & EDGERAG_ATTN_TILES_SHARED) != 0);
+                             (parts & EDGERAG_ATTN_TILES_SHARED) != 0,
+                             gqa ? decode_gqa_lds(D, ph[H_ROW_WAVES]) : 0);
       } else {
         dispatch_rows_qr<T, D>(a, 8, n_row, n_items - n_row, H_N_ITEMS);
       }
@@ -942,8 +947,6 @@ int run_items(const Launch& a, const int32_t* ph, int parts) {
       dispatch_rows_qr<T, D>(a, 8, n_row, n_items - n_row, H_N_ITEMS);
     }
   }
-  const int qr = std::min(8, pow2_at_least(std::max(1, ph[H_MAX_ROW_VECS])));
-  const bool fast = a.bs % C::TPW == 0 && ph[H_MAX_SPLIT_BLOCKS] <= kMaxSplitBlocks;
   if ((parts & EDGERAG_ATTN_ROWS) && n_row > 0) {
     if (fast)
       dispatch_decode_qr<T, D>(a, qr, 0, n_row, H_N_ROW_ITEMS, ph[H_ROW_WAVES], n_items > n_row);
@@ -1070,10 +1073,26 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
   // the rows, which also saves the host the fork and join of the streams. (Three 512-token
   // slices beside 24 decodes of up to 7,472 tokens, 707 MB of rows: 0.175 against 0.258 ms on
   // one stream. One 512-token chunk, 128 tiles, beside 7 decodes of 32-256 MB: every prefill
-  // iteration of the config-5 serving trace was faster on one stream.)
-  const bool overlap = n_tiles > 0 && row_items > 0 &&
-                       ((flags & EDGERAG_PLAN_OVERLAP) ||
-                        (n_tiles >= kPlanCUs && work * head_dim * 2 * es >= kOverlapRowBytes));
+  // iteration of the config-5 serving trace was faster on one stream.) Two kinds of batch gain
+  // nothing beside each other and stay on one stream, us on two / one: fp32, but for
+  // grouped rows in parts of contexts (two 300-token slices, 32/32 heads of 64 beside 12 decodes of
+  // 4,096 tokens 220 / 181, 32/8 of 64 with 48 of 6,000 274 / 246, 16/16 of 128 with 8 of 4,096 155 /
+  // 142; in parts 32/8 of 128 with 24 of 4,096 249 / 274, 32/8 of 64 142 / 141), and bf16 tiles of head_dim 128 beside rows of
+  // the VALU kernel, whose fp32 queries want the registers (32/32 heads, two 512-token slices, 8 of
+  // 4,096 225 / 214, 24 of 1,500 213 / 194; fp16 160 / 209, 174 / 182).
+  int64_t max_vecs = 0;  // most query vectors of a row
+  for (int r = 0; r < num_reqs; ++r) {
+    const int64_t v = (int64_t(query_start_loc[r + 1]) - query_start_loc[r]) * n_rep;
+    if (v <= kMaxRowVecs) max_vecs = std::max(max_vecs, v);
+  }
+  const bool valu_rows = !decode_gqa_shape(dtype, head_dim, int(max_vecs), block_size);
+  const bool one_stream =
+      (tile_kind > 1 && (row_items >= kPlanCUs || n_rep == 1)) ||
+      (tile_kind == 1 && dtype == EDGERAG_BF16 && head_dim == 128 && valu_rows);
+  const bool overlap =
+      n_tiles > 0 && row_items > 0 &&
+      ((flags & EDGERAG_PLAN_OVERLAP) ||
+       (!one_stream && n_tiles >= kPlanCUs && work * head_dim * 2 * es >= kOverlapRowBytes));
   // Batches with fewer row workgroups than CUs (one or a few long decodes: 32 workgroups for a
   // single request of 32 kv heads) instead cut every context into parts, one workgroup each, so
   // that about kRowTargetWgs workgroups cover the chip; a context's parts write fp32 partials
@@ -1088,13 +1107,7 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
       overlap && row_items >= kPlanCUs ? EDGERAG_ROW_WG_PART_TILES : EDGERAG_ROW_WG_PART,
       int64_t(kMaxSplitBlocks) * block_size);
   // Rows of 2 to 8 query vectors run on the GQA kernel (attention_decode_gqa.hip).
-  int64_t max_vecs = 0;
-  for (int r = 0; r < num_reqs; ++r) {
-    const int64_t v = (int64_t(query_start_loc[r + 1]) - query_start_loc[r]) * n_rep;
-    if (v <= kMaxRowVecs) max_vecs = std::max(max_vecs, v);
-  }
-  const bool gqa_rows =
-      head_dim == 128 && decode_gqa_shape(dtype, head_dim, int(max_vecs), block_size);
+  const bool gqa_rows = head_dim == 128 && !valu_rows;
   const int full_waves = gqa_rows ? kGqaWaves : kRowWgWaves;
   const int part_waves = gqa_rows ? kGqaWaves : kRowPartWaves;
   const int64_t part_cap =

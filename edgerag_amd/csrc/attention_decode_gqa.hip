@@ -539,6 +539,10 @@ bool decode_gqa_supported(const AttnLaunch& a, int32_t dtype, int32_t head_dim, 
          int64_t(a.nb) * a.bs * head_dim * 2 < int64_t(kOutOfRange);
 }
 
+unsigned decode_gqa_lds(int32_t head_dim, int waves) {
+  return unsigned(waves > 4 ? waves : 4) * 2 * kKeys * head_dim * 2;
+}
+
 void launch_decode_gqa(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int base, int count,
                        int limit_word, int vecs, int waves) {
   const bool half = dtype == EDGERAG_F16;

@@ -87,9 +87,10 @@ struct AttnLaunch {
 // Virtual query rows (token x head-in-group) per MFMA tile workgroup: 32 per wave.
 constexpr int kMfmaTileRows = EDGERAG_TILE_ROWS;
 constexpr int kMaxTileBlocks = 512;  // block ids one tile item stages in LDS (caps its split)
-// shared: one workgroup per CU (the rest of each CU is left to concurrently running rows).
+// shared: one workgroup per CU (the rest of each CU is left to concurrently running rows, if the
+// row_lds bytes of LDS that they need fit there).
 void launch_prefill_tiles(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int item_base,
-                          int count, bool shared);
+                          int count, bool shared, unsigned row_lds);
 // Whether the MFMA tile kernel is built for this element type and head_dim.
 bool prefill_tile_shape(int32_t dtype, int32_t head_dim);
 // Whether a pool of this size can use it (buffer-resource addressing).
@@ -103,6 +104,8 @@ constexpr int kGqaWaves = 4;  // waves of a workgroup row of the GQA kernel at h
 bool decode_gqa_shape(int32_t dtype, int32_t head_dim, int vecs, int32_t block_size);
 bool decode_gqa_supported(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int vecs,
                           int waves, bool tiles);
+// LDS of its rows that puts a wave on each SIMD of a CU (or one workgroup, if that is more).
+unsigned decode_gqa_lds(int32_t head_dim, int waves);
 void launch_decode_gqa(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int base, int count,
                        int limit_word, int vecs, int waves);
 // Prefill tiles in fp32 (attention_prefill_f32.hip), head_dim 64 and 128: 16 or 32 virtual rows.

@@ -73,7 +73,7 @@ constexpr int kThreads = kWaves * kWave;
 // below it).
 constexpr uint32_t kOutOfRange = 0xFFFFF000u;
 
-constexpr unsigned tile_lds(int d) { return 4 * kKeys * d * 2 + kMaxTileBlocks * 4; }
+constexpr unsigned tile_lds(int d) { return 4 * kKeys * d * 2 + kMaxTileBlocks * 4 + 24; }
 static_assert(tile_lds(64) + kSharedLdsPad <= 160 * 1024 &&
                   2 * (tile_lds(64) + kSharedLdsPad) > 160 * 1024 &&
                   tile_lds(128) + kSharedLdsPad <= 160 * 1024 &&
@@ -658,11 +658,19 @@ void attn_prefill_mfma_kernel(
 }
 
 template <typename T, int D>
-void launch_tiles(const AttnLaunch& a, int item_base, int count, bool shared) {
+void launch_tiles(const AttnLaunch& a, int item_base, int count, bool shared, unsigned row_lds) {
   // Shared mode reserves unused dynamic LDS so that a second workgroup no longer fits a CU's
   // 160 KiB (the static arrays take 34 or 66 KiB): the tiles then hold one of each SIMD's two
-  // register halves and decode waves keep the other.
-  const unsigned pad = shared ? kSharedLdsPad : 0;
+  // register halves and decode waves keep the other. Rows on the grouped kernel need LDS of
+  // their own (row_lds, for a wave per SIMD): where that does not fit beside tile and pad, the pad
+  // would hold the place of a second tile for rows that cannot use it, and is left out (the rows
+  // then fill in as tiles end). Slices beside decodes, us with the pad / without: bf16 32/8 heads
+  // of 128, two at 4,096 keys with 24 of 4,096 tokens 194 / 158, with 60 of 1,200 168 / 143, with 40
+  // of 2,000 145 / 151; 32/8 of 64, three with 32 of 8,000 (rows of 16 waves) 195 / 161. Where
+  // it fits (rows of 8 waves or one wave at 64): three with 20 of 8,192 115 / 131, with 48 of
+  // 4,096 132 / 140, of 8,000 211 / 199.
+  const bool fits = tile_lds(D) + kSharedLdsPad + row_lds <= 160 * 1024;
+  const unsigned pad = shared && fits ? kSharedLdsPad : 0;
   hipLaunchKernelGGL((attn_prefill_mfma_kernel<T, D>), dim3(count), dim3(kThreads), pad, a.s,
                      a.plan, item_base, log2_exact(a.bs), a.qsl, a.ctx, a.bt, a.bt_stride, a.nb,
                      a.hq, static_cast<const T*>(a.q), a.q_st, a.q_sh,
@@ -683,14 +691,14 @@ bool prefill_tiles_supported(int32_t num_blocks, int32_t block_size, int32_t hea
 }
 
 void launch_prefill_tiles(const AttnLaunch& a, int32_t dtype, int32_t head_dim, int item_base,
-                          int count, bool shared) {
+                          int count, bool shared, unsigned row_lds) {
   const bool half = dtype == EDGERAG_F16;
   if (head_dim == 64) {
-    if (half) launch_tiles<f16, 64>(a, item_base, count, shared);
-    else launch_tiles<bf16, 64>(a, item_base, count, shared);
+    if (half) launch_tiles<f16, 64>(a, item_base, count, shared, row_lds);
+    else launch_tiles<bf16, 64>(a, item_base, count, shared, row_lds);
   } else {
-    if (half) launch_tiles<f16, 128>(a, item_base, count, shared);
-    else launch_tiles<bf16, 128>(a, item_base, count, shared);
+    if (half) launch_tiles<f16, 128>(a, item_base, count, shared, row_lds);
+    else launch_tiles<bf16, 128>(a, item_base, count, shared, row_lds);
   }
 }
 

@@ -145,7 +145,9 @@ int edgerag_attn_plan(const int32_t* query_start_loc, const int32_t* context_len
  * plan word 20 (1: two streams, 0: one): the tiles (EDGERAG_ATTN_TILES | EDGERAG_ATTN_TILES_SHARED)
  * on one stream beside the rows (EDGERAG_ATTN_ROWS) on another, joined before
  * EDGERAG_ATTN_COMBINE; or EDGERAG_ATTN_ALL on one stream. The planner picks two streams when the
- * tiles fill every CU at one workgroup each and the rows read at least 256 MiB of K/V;
+ * tiles fill every CU at one workgroup each and the rows read at least 256 MiB of K/V (in fp32 only
+ * for grouped heads and few decodes, in bf16 at head_dim 128 only for grouped heads: the others
+ * gain nothing);
  * EDGERAG_PLAN_OVERLAP asks for it whenever the batch holds both. Either run of either plan gives
  * the same results; the plan only sizes the work items for the run it names.
  */
@@ -177,8 +179,8 @@ int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_t* context_
  *   EDGERAG_ATTN_ALL      all three in order on `stream`.
  * Tiles and rows write disjoint outputs and partials. EDGERAG_ATTN_TILES_SHARED, added to
  * EDGERAG_ATTN_TILES, runs the MFMA tiles at one workgroup per CU, which leaves the rest of every
- * CU's registers to decode rows enqueued on another stream; enqueue the tiles first. It changes
- * nothing in the results.
+ * CU's registers to decode rows enqueued on another stream (where the rows' LDS fits there too, else
+ * the tiles run as without it); enqueue the tiles first. It changes nothing in the results.
  */
 int edgerag_paged_attention(const int32_t* plan_host, const int32_t* plan_dev, int64_t plan_words,
                             const void* q, int64_t q_stride_tok, int64_t q_stride_head,

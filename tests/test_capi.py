@@ -453,6 +453,23 @@ def test_wide_tile_partials_fit_the_static_scratch(n_q, n_kv) -> None:
             assert all(int(reqs[r][1]) % 64 == 0 for r in range(n))
 
 
+@pytest.mark.parametrize("dtype,n_q,n_kv,d,n,overlap", [
+    (torch.float32, 32, 32, 64, 40, 0), (torch.float32, 32, 8, 64, 40, 0),
+    (torch.float32, 32, 8, 64, 24, 1), (torch.float32, 16, 16, 128, 8, 0),
+    (torch.bfloat16, 32, 32, 128, 40, 0), (torch.float16, 32, 32, 128, 40, 1),
+    (torch.bfloat16, 32, 8, 128, 40, 1), (torch.float16, 32, 8, 128, 40, 1),
+    (torch.bfloat16, 32, 32, 64, 40, 1), (torch.bfloat16, 32, 8, 64, 40, 1),
+])
+def test_plan_overlap_only_where_rows_run_beside_the_tiles(dtype, n_q, n_kv, d, n, overlap) -> None:
+    """Heavy slices beside heavy decodes take two streams only in the types and head dims where they
+    measured faster for it; a forced plan takes them anyway."""
+    qsl, ctx = _mixed([(512, 3000)] * 4, [6000] * n)
+    for force in (False, True):
+        plan, _ = kernels.make_plan_host(qsl, ctx, n_q, n_kv, d, 16, 400, dtype,
+                                         force_overlap=force)
+        assert int(plan[20]) == (1 if force else overlap)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("n_q,n_kv", [(32, 32), (32, 8)])
