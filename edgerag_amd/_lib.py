@@ -36,6 +36,8 @@ ATTN_TILES, ATTN_ROWS, ATTN_COMBINE, ATTN_ALL = 1, 2, 4, 7
 ATTN_TILES_SHARED = 8  # modifier of ATTN_TILES: one tile workgroup per CU, beside decode rows
 PLAN_SPLIT_ROWS = 1  # edgerag_attn_plan_ex flag: decode rows as KV splits merged by a launch
 PLAN_OVERLAP = 2  # edgerag_attn_plan_ex flag: plan tiles beside rows (two streams) whenever both
+PLAN_WORKSPACE = 4  # edgerag_attn_plan_ex flag: splits may need more than the static scratch
+PLAN_WORD_FITS_SCRATCH = 22  # plan word: 1 when the batch fits the scratch without PLAN_WORKSPACE
 PLAN_WORD_OVERLAP = 20  # plan word: 1 when the plan is for tiles and rows on two streams
 QUANT_WORKSPACE_MAX = 8 * 1024 * 1024  # bound of edgerag_quant_linear_workspace_bytes
 ATTN_SCRATCH_BYTES = 32 * 1024 * 1024  # static partials of edgerag_paged_attention_noalloc

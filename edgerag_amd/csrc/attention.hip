@@ -981,7 +981,7 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
                                     int32_t* plan, int64_t plan_capacity_words,
                                     int64_t* plan_words, int64_t* workspace_bytes) {
   clear_error();
-  if ((flags & ~(EDGERAG_PLAN_SPLIT_ROWS | EDGERAG_PLAN_OVERLAP)) != 0)
+  if ((flags & ~(EDGERAG_PLAN_SPLIT_ROWS | EDGERAG_PLAN_OVERLAP | EDGERAG_PLAN_WORKSPACE)) != 0)
     return fail(EDGERAG_EINVAL, "edgerag_attn_plan: flags %d", flags);
   if (plan_words == nullptr || workspace_bytes == nullptr)
     return fail(EDGERAG_EINVAL, "edgerag_attn_plan: plan_words/workspace_bytes are NULL");
@@ -1179,10 +1179,15 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
   // one tile per CU whose tiles hold p in 32 bits (bf16, or head_dim 128) aim at kTargetTiles / 2
   // as well: the partials of twice the items cost more than the second workgroup per CU gains (512
   // tokens at 3,072 keys: fp16 32/8 heads of 128 65.3 -> 62.0 us, bf16 32/32 of 64 43.3 -> 40.9;
-  // bf16 32/8 of 128, slices at 2,048 and 4,096: 139 -> 128 us).
+  // bf16 32/8 of 128, slices at 2,048 and 4,096: 139 -> 128 us). So do larger batches at head_dim
+  // 128 in 16 bits, where halves of 384 tiles cost more than a second, half-filled round of whole ones
+  // (three 512-token slices at 4,096 keys, 768 / 384 items: bf16 32/8 heads 169 / 156 us, fp16 32/32
+  // 188 / 172).
   // A split may span at most kMaxTileBlocks blocks (the MFMA tile kernel stages its block ids).
-  const int64_t target_tiles =
-      overlap || (wide_tiles && n_tiles <= kPlanCUs) ? kTargetTiles / 2 : kTargetTiles;
+  const bool wide_128 = tile_kind == 1 && head_dim == 128;
+  const int64_t target_tiles = overlap || wide_128 || (wide_tiles && n_tiles <= kPlanCUs)
+                                   ? kTargetTiles / 2
+                                   : kTargetTiles;
   const int64_t tile_split_cap =
       std::max<int64_t>(64, int64_t(kMaxTileBlocks - 1) * block_size / 64 * 64);
   const int64_t tile_share = round_up(
@@ -1192,8 +1197,8 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
                           ? tile_share
                           : round_up(std::max<int64_t>(max_len, 1), 64));
   // Keys of a tile request's splits: equal 64-key multiples of at most tile_part.
-  auto tile_split_len = [&](int64_t L) -> int64_t {
-    const int64_t n = std::max<int64_t>(1, (L + tile_part - 1) / tile_part);
+  auto tile_split_len = [&](int64_t L, int64_t part) -> int64_t {
+    const int64_t n = std::max<int64_t>(1, (L + part - 1) / part);
     return std::min(tile_split_cap, round_up((std::max<int64_t>(L, 1) + n - 1) / n, 64));
   };
 
@@ -1202,29 +1207,38 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
     int64_t len;
     int n, pstride;
   };
-  auto request_split = [&](int64_t c, int64_t L) -> RequestSplit {
+  auto request_split = [&](int64_t c, int64_t L, int64_t part) -> RequestSplit {
     const bool row = c * n_rep <= kMaxRowVecs;
     // Workgroup-split rows: one item per part of the context (the waves split the part).
-    const int64_t slen = row ? (wg_rows ? wg_split_len(L) : split_len) : tile_split_len(L);
+    const int64_t slen = row ? (wg_rows ? wg_split_len(L) : split_len) : tile_split_len(L, part);
     const int n = c == 0 ? 0 : int((L + slen - 1) / slen);
     // Slotted row requests write partials (and get merge rows) even when not split.
     return {slen, n, slots > 0 && row ? slots : n};
   };
   // The partials of the wide tiles (128 rows of head_dim 128 take 66 KB a split) fit the static
   // scratch of edgerag_paged_attention_noalloc wherever longer splits make them fit: past it,
-  // tiles are split less. (fp16 head_dim 64 plans keep their splits.)
+  // tiles are split less. (fp16 head_dim 64 plans keep their splits.) A plan for a workspace
+  // keeps the splits that fill the chip (bf16 64/8 heads of 128, 256 tokens at 4,096 keys beside 24
+  // decodes of 4,096: 24 MB of them the rows', 153 us against 178 in tiles of whole contexts), and
+  // so does one whose decode rows alone leave no room; H_FITS_SCRATCH says which could have fit.
+  int fits_scratch = 0;
   if (wide_tiles) {
-    auto partial_bytes = [&] {
+    auto partial_bytes = [&](int64_t part) {
       int64_t n = 0;
       for (int r = 0; r < num_reqs; ++r) {
         const int64_t c = int64_t(query_start_loc[r + 1]) - query_start_loc[r];
-        const RequestSplit rs = request_split(c, context_lens[r]);
+        const RequestSplit rs = request_split(c, context_lens[r], part);
         if (c > 0 && rs.pstride > 1) n += c * n_q_heads * rs.pstride;
       }
       return workspace_layout(n, head_dim).total;
     };
-    while (tile_part < tile_split_cap && partial_bytes() > EDGERAG_ATTN_SCRATCH_BYTES)
-      tile_part = std::min(tile_split_cap, 2 * tile_part);
+    int64_t part = tile_part, bytes = partial_bytes(part);
+    while (part < tile_split_cap && bytes > EDGERAG_ATTN_SCRATCH_BYTES) {
+      part = std::min(tile_split_cap, 2 * part);
+      bytes = partial_bytes(part);
+    }
+    fits_scratch = bytes <= EDGERAG_ATTN_SCRATCH_BYTES;
+    if (fits_scratch && !(flags & EDGERAG_PLAN_WORKSPACE)) tile_part = part;
   }
 
   // Scratch reused across calls on a thread: the planner runs once per step on the host.
@@ -1242,7 +1256,7 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
     const int L = context_lens[r];
     int32_t* rq = reqs.data() + size_t(r) * kReqWords;
     const bool row = c * n_rep <= kMaxRowVecs;
-    const RequestSplit rs = request_split(c, L);
+    const RequestSplit rs = request_split(c, L, tile_part);
     const int64_t slen = rs.len;
     const int nsplit = rs.n, pstride = rs.pstride;
     const bool slotted = slots > 0 && row;
@@ -1319,6 +1333,7 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
   plan[H_ROW_WAVES] = row_waves;
   plan[H_OVERLAP] = overlap ? 1 : 0;
   plan[H_SLOTS] = slots;
+  plan[H_FITS_SCRATCH] = fits_scratch;
   std::copy(combine.begin(), combine.end(), plan + combine_off);
   int32_t* dst = plan + item_off;
   for (const auto* groups : {&rows, &tiles})

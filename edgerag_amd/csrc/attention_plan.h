@@ -41,6 +41,8 @@ enum Header {
   H_OVERLAP,           // 1: planned for tiles and rows on two streams (tiles shared), 0: one
   H_SLOTS,             // S > 0: the row requests' partials sit in S slots per (token, q head)
                        // (rows cut into parts); 0: nsplit slots per (token, q head)
+  H_FITS_SCRATCH,      // 1: of wide tiles, and planned without EDGERAG_PLAN_WORKSPACE the partials
+                       // fit the static scratch
 };
 // Waves a workgroup-split row item may use (the kernel's LDS merge is sized for this many).
 constexpr int kMaxRowWaves = 16;

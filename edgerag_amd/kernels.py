@@ -256,6 +256,7 @@ def make_plan_host(
     dtype: torch.dtype,
     split_rows: bool = False,
     force_overlap: bool = False,
+    workspace: bool = False,
 ) -> tuple[np.ndarray, int]:
     """Run the native host planner. Returns ``(plan words, workspace bytes)``.
 
@@ -264,7 +265,8 @@ def make_plan_host(
     plans decode rows as KV splits merged by a launch (``EDGERAG_PLAN_SPLIT_ROWS``) instead of
     workgroups whose waves merge in LDS. ``force_overlap`` plans any batch with both prefill
     tiles and decode rows for the two-stream run (``EDGERAG_PLAN_OVERLAP``), which the planner
-    otherwise picks only when both are heavy."""
+    otherwise picks only when both are heavy. ``workspace``: the plan runs with a workspace, so its
+    tile splits need not fit the static scratch (``EDGERAG_PLAN_WORKSPACE``)."""
     lib = _lib.load()
     qsl = np.ascontiguousarray(query_start_loc, dtype=np.int32)
     ctx = np.ascontiguousarray(context_lens, dtype=np.int32)
@@ -275,7 +277,8 @@ def make_plan_host(
     args = (
         qsl.ctypes.data, ctx.ctypes.data, num_reqs, n_q_heads, n_kv_heads, head_dim, block_size,
         max_blocks_per_seq, dtype_code(dtype),
-        (_lib.PLAN_SPLIT_ROWS if split_rows else 0) | (_lib.PLAN_OVERLAP if force_overlap else 0),
+        (_lib.PLAN_SPLIT_ROWS if split_rows else 0) | (_lib.PLAN_OVERLAP if force_overlap else 0)
+        | (_lib.PLAN_WORKSPACE if workspace else 0),
     )
     plan = np.empty(_PLAN_WORDS_HINT[0], dtype=np.int32)
     rc = lib.edgerag_attn_plan_ex(*args, plan.ctypes.data, plan.size, ctypes.byref(words),
@@ -317,7 +320,7 @@ def plan_attention(
         raise ValueError("block_tables must be (num_reqs, max_blocks)")
     plan, ws_bytes = make_plan_host(
         query_start_loc, context_lens, n_q_heads, n_kv_heads, head_dim, block_size,
-        block_tables.shape[1], dtype, split_rows, force_overlap,
+        block_tables.shape[1], dtype, split_rows, force_overlap, workspace,
     )
     extra = list(extra_int32 or [])
     views = upload_int32(
@@ -427,10 +430,18 @@ def paged_attention_noalloc(
     """:func:`paged_attention` through ``edgerag_paged_attention_noalloc``: the split partials
     live in the library's static per-GPU scratch (``_lib.ATTN_SCRATCH_BYTES``), so the call
     allocates nothing, ``out`` included (the caller passes it). Calls that overlap in time on one
-    GPU share that scratch and must be ordered by the caller (one stream does it)."""
+    GPU share that scratch and must be ordered by the caller (one stream does it). A plan that was
+    split further because it has a workspace of its own (``workspace=False`` would have fit the
+    scratch) keeps its partials there."""
     if out is None:
         raise ValueError("paged_attention_noalloc writes into a caller-provided out")
     query, out, lead = _attention_operands(query, key_pool, value_pool, plan, out)
+    if (plan.workspace is not None and plan.workspace_bytes > _lib.ATTN_SCRATCH_BYTES
+            and plan.plan_host[_lib.PLAN_WORD_FITS_SCRATCH]):
+        call("edgerag_paged_attention", *lead, float(scale), out.data_ptr(), out.stride(0),
+             out.stride(1), plan.workspace.data_ptr(), plan.workspace_bytes, int(parts),
+             stream_ptr(query.device))
+        return out
     call("edgerag_paged_attention_noalloc", *lead, float(scale), out.data_ptr(), out.stride(0),
          out.stride(1), int(parts), stream_ptr(query.device))
     return out

@@ -150,9 +150,15 @@ int edgerag_attn_plan(const int32_t* query_start_loc, const int32_t* context_len
  * gain nothing);
  * EDGERAG_PLAN_OVERLAP asks for it whenever the batch holds both. Either run of either plan gives
  * the same results; the plan only sizes the work items for the run it names.
+ *
+ * Prefill tiles in bf16, fp32 or of head_dim 128 are split over the keys only as far as the batch's
+ * partials fit EDGERAG_ATTN_SCRATCH_BYTES, where fewer splits make them fit, so that the plan serves
+ * edgerag_paged_attention_noalloc too. EDGERAG_PLAN_WORKSPACE lifts that for a plan that runs with a
+ * workspace of the reported size; plan word 22 then says whether the batch would have fit without.
  */
 #define EDGERAG_PLAN_SPLIT_ROWS 1
 #define EDGERAG_PLAN_OVERLAP 2
+#define EDGERAG_PLAN_WORKSPACE 4
 int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_t* context_lens,
                          int32_t num_reqs, int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,
                          int32_t block_size, int32_t max_blocks_per_seq, int32_t dtype,

@@ -453,6 +453,31 @@ def test_wide_tile_partials_fit_the_static_scratch(n_q, n_kv) -> None:
             assert all(int(reqs[r][1]) % 64 == 0 for r in range(n))
 
 
+@pytest.mark.parametrize("n_q,c,n,L", [(64, 256, 24, 4096), (64, 256, 64, 8192),
+                                       (64, 128, 100, 8192), (32, 512, 128, 8192),
+                                       (64, 256, 128, 8192)])
+def test_decode_rows_leave_the_splits_of_a_workspace_plan(n_q, c, n, L) -> None:
+    """Decode rows' partials beside a slice take none of its splits in a plan that runs with a
+    workspace: the tiles fill the chip as they do beside 7 decodes. Without the flag the plan fits
+    the no-alloc entry's scratch with fewer splits, or keeps them where the rows alone fill it;
+    plan word 22 says which."""
+    def plan(decodes, workspace):
+        qsl, ctx = _mixed([(c, 4096 - c)], [L] * decodes)
+        words, nbytes = kernels.make_plan_host(qsl, ctx, n_q, 8, 128, 16, 512, torch.bfloat16,
+                                               workspace=workspace)
+        return words, int(words[2]) - int(words[13]), nbytes
+
+    _few, tiles, _ = plan(7, True)
+    assert tiles >= 256
+    free, free_tiles, free_bytes = plan(n, True)
+    assert free_tiles == tiles and free_bytes > _lib.ATTN_SCRATCH_BYTES
+    words, fit_tiles, nbytes = plan(n, False)
+    assert int(free[22]) == int(words[22]) == int(nbytes <= _lib.ATTN_SCRATCH_BYTES)
+    assert fit_tiles < tiles if words[22] else fit_tiles == tiles
+    qsl, ctx = _mixed([(c, 4096 - c)], [L] * n)
+    assert kernels.make_plan_host(qsl, ctx, 32, 8, 64, 16, 512, torch.float16)[0][22] == 0
+
+
 @pytest.mark.parametrize("dtype,n_q,n_kv,d,n,overlap", [
     (torch.float32, 32, 32, 64, 40, 0), (torch.float32, 32, 8, 64, 40, 0),
     (torch.float32, 32, 8, 64, 24, 1), (torch.float32, 16, 16, 128, 8, 0),

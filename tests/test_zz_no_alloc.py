@@ -123,3 +123,28 @@ def test_noalloc_refuses_plans_beyond_the_scratch() -> None:
     assert rc == _lib.EDGERAG_EWORKSPACE
     msg = lib.edgerag_last_error().decode()
     assert "static scratch holds" in msg and str(_lib.ATTN_SCRATCH_BYTES) in msg
+
+
+@pytest.mark.gpu
+def test_noalloc_takes_a_workspace_plan_that_would_have_fit(device) -> None:
+    """A plan made for a workspace may be split further than the scratch holds. Where the batch fits
+    without that (24 decodes beside a 256-token slice, bf16, 64/8 heads of 128), the no-alloc call
+    takes either plan: the one without a workspace in the scratch, the other in its own workspace."""
+    lens = np.asarray([4096] * 25, np.int32)
+    qsl = np.concatenate([[0], 256 + np.arange(25)]).astype(np.int32)
+    nb = 25 * 256
+    bt = np.random.RandomState(7).permutation(nb).astype(np.int32).reshape(25, 256)
+    g = torch.Generator(device=device).manual_seed(7)
+    kp, vp = (torch.randn((8, nb, BS, 128), generator=g, device=device, dtype=torch.bfloat16)
+              for _ in range(2))
+    q = torch.randn((280, 64, 128), generator=g, device=device, dtype=torch.bfloat16)
+    outs = []
+    for workspace in (True, False):
+        plan, _ = kernels.plan_attention(qsl, lens, bt, 64, 8, 128, BS, torch.bfloat16, device,
+                                         workspace=workspace)
+        assert (plan.workspace_bytes > _lib.ATTN_SCRATCH_BYTES) == workspace
+        outs.append(kernels.paged_attention_noalloc(q, kp, vp, plan, 128**-0.5,
+                                                    torch.full_like(q, float("nan"))))
+    torch.testing.assert_close(outs[0], outs[1], rtol=2.0**-7, atol=2.0**-12)  # bf16 neighbours
+    ws = kernels.plan_attention(qsl, lens, bt, 64, 8, 128, BS, torch.bfloat16, device)[0]
+    assert torch.equal(kernels.paged_attention(q, kp, vp, ws, 128**-0.5, overlap=False), outs[0])
