@@ -51,6 +51,7 @@ typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 #ifndef EDGERAG_ATTN_SHARED_PAD_KB
 #define EDGERAG_ATTN_SHARED_PAD_KB 48  // dynamic LDS of a shared-mode tile workgroup
@@ -186,6 +187,15 @@ __device__ __forceinline__ void load_lds16(Slice s, char* dst, uint32_t off) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(
       __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(s.base), 0, s.bytes, 0x00020000),
       (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
+}
+
+// 16 bytes of the slice at byte offset row + in_row (zeros past its end).
+__device__ __forceinline__ u32x4 load16(Slice s, uint32_t row, int in_row) {
+  return __builtin_bit_cast(
+      u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                 __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(s.base), 0, s.bytes,
+                                                   0x00020000),
+                 __builtin_elementwise_add_sat(row, uint32_t(in_row)), 0, 0));
 }
 
 // One wave's share of a tile: load j fills the 64 / (D / 8) rows at dst + 1024 j lane by lane,
@@ -583,41 +593,51 @@ void attn_prefill_mfma_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) any_odd = __builtin_fmaf(o[dt][i], 0.f, any_odd);
   if (__any(active && any_odd != 0.f)) {
+    // (Loads through the descriptors of the main loop, and indexes of this lane formed here: nothing
+    // of this is held in registers across the loop.)
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
     auto row_of = [&](int pos) {  // byte offset of key pos in the head's slice
       return __builtin_elementwise_add_sat(sblk[(pos >> bs_shift) - geo.blk0],
                                            uint32_t(pos & geo.bs_mask) * uint32_t(D * 2));
     };
-    auto finite = [](T v) { return __builtin_fabsf(to_f32<T>(v)) < INFINITY; };
     bool hidden = false;  // a non-finite V among the keys that some row of the wave does not see
-    for (int pos = max(kb, wave_min_lim + 1) + lane / kCh; pos < ke; pos += kKpi) {
-      const uint32_t off = row_of(pos);
-      const T* v = reinterpret_cast<const T*>(static_cast<const char*>(vrs.base) + off);
-      for (int e = 0; e < 8; ++e) hidden |= off < vrs.bytes && !finite(v[8 * (lane % kCh) + e]);
+    for (int pos = max(kb, wave_min_lim + 1) + ln / kCh; pos < ke; pos += kKpi) {
+      const v8 v = __builtin_bit_cast(v8, load16(vrs, row_of(pos), 16 * (ln % kCh)));
+#pragma unroll
+      for (int e = 0; e < 8; ++e) hidden |= !(__builtin_fabsf(float(v[e])) < INFINITY);
     }
     if (__any(hidden)) {
-      const T* qp = sq.q + int64_t(t) * sq.st + int64_t(hq) * sq.sh;
+      const T* qp = sq.q + int64_t(t) * sq.st + int64_t(hq) * sq.sh + 8 * (ln / 32);
 #pragma unroll
       for (int dt = 0; dt < kDt; ++dt) o[dt] = f32x16{};
       for (int pos = kb; pos < ke; ++pos) {
         const uint32_t off = row_of(pos);
-        if (off >= vrs.bytes) continue;
-        const T* k = reinterpret_cast<const T*>(static_cast<const char*>(krs.base) + off);
-        const T* v = reinterpret_cast<const T*>(static_cast<const char*>(vrs.base) + off);
+        if (off >= krs.bytes) continue;
         float s = 0.f;
-        for (int ks = 0; ks < kKs; ++ks)
 #pragma unroll
-          for (int e = 16 * ks + 8 * g; e < 16 * ks + 8 * g + 8; ++e)
-            s = __builtin_fmaf(to_f32<T>(qp[e]), to_f32<T>(k[e]), s);
+        for (int ks = 0; ks < kKs; ++ks) {
+          const v8 k = __builtin_bit_cast(v8, load16(krs, off, 32 * ks + 16 * (ln / 32)));
+          const v8 qk = *reinterpret_cast<const v8*>(qp + 16 * ks);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) s = __builtin_fmaf(float(qk[e]), float(k[e]), s);
+        }
         float p = exp2_fast(__builtin_fmaf(halves_sum(s), scale_log2, nm));
         if constexpr (!kSplit)
           p = float(__builtin_bit_cast(h2, E::head_rtz(f2{p, 0.f}))[0]);
         if (pos > lim) continue;
+        // Dims 32 dt + 8 qd + 0-3 (lanes of the lower half) and + 4-7 (of the upper).
 #pragma unroll
         for (int dt = 0; dt < kDt; ++dt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i)
-            o[dt][i] = __builtin_fmaf(
-                p, to_f32<T>(v[32 * dt + (i & 3) + 8 * (i >> 2) + 4 * g]), o[dt][i]);
+          for (int qd = 0; qd < 4; ++qd) {
+            const v8 v = __builtin_bit_cast(v8, load16(vrs, off, 64 * dt + 16 * qd));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float ve = ln < 32 ? float(v[e]) : float(v[4 + e]);
+              o[dt][4 * qd + e] = __builtin_fmaf(p, ve, o[dt][4 * qd + e]);
+            }
+          }
       }
     }
   }
