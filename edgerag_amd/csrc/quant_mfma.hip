@@ -15,8 +15,8 @@
 //   Only the lane-to-k assignment inside a k-step differs from textbook order, identically for
 //   both operands: INT4 nibbles decode to the k order (0,4,1,5,2,6,3,7), so the activations are
 //   permuted the same way in registers.
-// * qlinear_gemm_kernel (M > 64, prefill slices): MFMA-bound. A 256-thread workgroup computes a
-//   BN x BM tile of y^T through v_mfma_f32_32x32x16_f16; per 64-k step it stages the dequantised
+// * qlinear_gemm_kernel (M > 64, prefill slices): MFMA-bound. A workgroup of 256 (or, of
+//   the 128x256 and 256x256 tiles, 512) threads computes a BN x BM tile of y^T through v_mfma_f32_32x32x16_f16; per 64-k step it stages the dequantised
 //   weights and the activations in double-buffered, XOR-swizzled LDS, loading the next steps'
 //   bytes from global memory while the current one is computed. With a workspace
 //   (edgerag_quant_linear_ws) it also takes decode batches past the streaming GEMV's crossover,
@@ -1634,11 +1634,12 @@ bool gemm_tiles_256(int32_t m, int32_t n) {
 //     8192 44.9 / 42.4, 4096 -> 6144 71.8 / 63.6, 2,048 rows 8192 -> 4096 159 / 142. A second round
 //     that is nearly empty costs little, and INT4 dequantises more a tile: 1,024 rows 4608 -> 4608,
 //     288 tiles, 80.7 / 86.4 (900 rows), 1,536 rows, 432 tiles, 95.2 / 91.1.
-//   * 128x128 for less than one round, where 128x64 tiles need a second: 128x64 / 128x128, us: 519
-//     rows 2048 -> 6144 25.1 / 23.0, 560 rows 2048 -> 4096 23.4 / 21.7, 1,536 rows 2048 -> 2048 24.9
-//     / 22.7. Only for INT8 layers of up to 12 M codes: a round of fewer, larger workgroups has fewer
-//     loads in flight, and past that the weights take longer (4096 -> 4096 at 640 rows 44.2 / 46.3,
-//     2048 -> 8192 at 384 rows 25.0 / 25.6; INT4 1152 -> 3456 at 640 rows 18.6 / 19.4).
+//   * INT8 128x128 for less than one round, where 128x64 tiles need a second and the last row of
+//     tiles is at least 16 rows short. Whole rows of 128x128 tiles are slower, whatever the layer;
+//     128x64 / 128x128, us, weights from memory as in a model: 2048 -> 4096 at 600 rows 23.8 / 23.2,
+//     704 24.0 / 23.3, 768 24.4 / 25.3; 2048 -> 6144 at 530 rows 25.2 / 23.6, 512 24.7 / 25.5; 4096 ->
+//     4096 at 576 rows 42.5 / 41.1, 610 42.7 / 41.7, 632 42.8 / 42.8, 639 43.2 / 46.4; 8192 -> 2048 at
+//     1,500 rows 83.7 / 78.7, 1,536 83.6 / 87.4. (INT4 1152 -> 3456 at 640 rows 18.6 / 19.4.)
 // Every tile sums in the same order: the same bits.
 enum class GemmTile { k64, k128x64, k128, k128x256, k256 };
 
@@ -1646,16 +1647,15 @@ inline int64_t gemm_tiles(int32_t m, int32_t n, int bm, int bn) {
   return int64_t((n + bn - 1) / bn) * ((m + bm - 1) / bm);
 }
 
-GemmTile gemm_tile(int32_t m, int32_t k, int32_t n, int bits) {
-  constexpr int64_t kCUs = EDGERAG_GEMM_TARGET_WGS, kCodes128 = int64_t(12) << 20;
+GemmTile gemm_tile(int32_t m, int32_t n, int bits) {
+  constexpr int64_t kCUs = EDGERAG_GEMM_TARGET_WGS;
   if (gemm_tiles_256(m, n)) return GemmTile::k256;
   const int64_t t128 = gemm_tiles(m, n, 128, 128), t128x64 = gemm_tiles(m, n, 64, 128);
   if (t128 > (bits == 8 ? kCUs : kCUs * 5 / 4) && gemm_tiles(m, n, 256, 128) <= kCUs)
     return GemmTile::k128x256;
   if (t128 >= kCUs) return GemmTile::k128;
   if (t128x64 < kCUs) return GemmTile::k64;
-  return bits == 8 && t128x64 > kCUs && int64_t(n) * k <= kCodes128 ? GemmTile::k128
-                                                                    : GemmTile::k128x64;
+  return bits == 8 && t128x64 > kCUs && (m - 1) % 128 < 112 ? GemmTile::k128 : GemmTile::k128x64;
 }
 
 // Rows past whole 64-row tiles (the decode tokens packed after a prefill chunk) that run on the
@@ -1665,13 +1665,13 @@ GemmTile gemm_tile(int32_t m, int32_t k, int32_t n, int bits) {
 // and without the last four, 46.2 against 40.6; 2048 -> 16384, 200 rows 32.6 against 24.5). 128x64
 // tiles (up to three workgroups per CU) take an extra row at almost no cost. 64x64 tiles always
 // pass them on, as the workspace route does (2048 -> 2048, 519 rows: 14.7 against 15.8).
-int gemm_remainder(int32_t m, int32_t k, int32_t n, int bits) {
+int gemm_remainder(int32_t m, int32_t n, int bits) {
   const int rem = m % 64;
   if (rem == 0 || rem > 16 || m - rem < 128) return 0;
-  const GemmTile tile = gemm_tile(m, k, n, bits);
+  const GemmTile tile = gemm_tile(m, n, bits);
   if (tile == GemmTile::k64) return rem;
   if (tile == GemmTile::k128x64) return 0;
-  if (gemm_tile(m - rem, k, n, bits) != tile)
+  if (gemm_tile(m - rem, n, bits) != tile)
     return tile == GemmTile::k128 && gemm_tiles(m, n, 128, 128) <= EDGERAG_GEMM_TARGET_WGS ? 0 : rem;
   const int bm = tile == GemmTile::k128 ? 128 : 256, bn = tile == GemmTile::k256 ? 256 : 128;
   auto rounds = [&](int32_t rows) {
@@ -1694,9 +1694,9 @@ bool stream_swiglu_shape(int32_t m, int32_t k, int32_t n) {
 // streaming path goes to the streaming SwiGLU kernel.
 bool gemm_swiglu_shape(int32_t m, int32_t k, int32_t n) {
   if (m <= EDGERAG_SKINNY_MAX_M || n % 2 != 0 || k % kBK != 0) return false;
-  if (const int rem = gemm_remainder(m, k, n, 8))
+  if (const int rem = gemm_remainder(m, n, 8))
     return gemm_swiglu_shape(m - rem, k, n) && stream_swiglu_shape(rem, k, n);
-  return gemm_tile(m, k, n, 8) != GemmTile::k64;
+  return gemm_tile(m, n, 8) != GemmTile::k64;
 }
 
 void dispatch_stream_swiglu(const f16* x, int64_t xs, int32_t m, int32_t k, const uint8_t* packed,
@@ -1706,13 +1706,13 @@ void dispatch_stream_swiglu(const f16* x, int64_t xs, int32_t m, int32_t k, cons
 void dispatch_gemm_swiglu(const f16* x, int64_t xs, int32_t m, int32_t k, const uint8_t* packed,
                           const f16* scales, const f16* bias, int32_t n, f16* y, int64_t ys,
                           hipStream_t s) {
-  if (const int rem = gemm_remainder(m, k, n, 8)) {
+  if (const int rem = gemm_remainder(m, n, 8)) {
     dispatch_gemm_swiglu(x, xs, m - rem, k, packed, scales, bias, n, y, ys, s);
     dispatch_stream_swiglu(x + int64_t(m - rem) * xs, xs, rem, k, packed, scales, bias, n,
                            y + int64_t(m - rem) * ys, ys, EpiArgs{}, s);
     return;
   }
-  const GemmTile tile = gemm_tile(m, k, n, 8);
+  const GemmTile tile = gemm_tile(m, n, 8);
   // 256x256 tiles hold four 32-row tiles a wave, which the epilogue does not pair: 128x256 ones
   // (2,048 rows 2048 -> 16384: 166 us on 128x128 tiles, 157 on these).
   if (tile == GemmTile::k128x256 || tile == GemmTile::k256)
@@ -1759,13 +1759,13 @@ void dispatch(const f16* x, int64_t xs, int32_t m, int32_t k, const uint8_t* pac
     }
     return;
   }
-  if (const int rem = gemm_remainder(m, k, n, BITS)) {
+  if (const int rem = gemm_remainder(m, n, BITS)) {
     dispatch<BITS>(x, xs, m - rem, k, packed, scales, bias, n, g, y, ys, s);
     dispatch<BITS>(x + int64_t(m - rem) * xs, xs, rem, k, packed, scales, bias, n, g,
                    y + int64_t(m - rem) * ys, ys, s);
     return;
   }
-  switch (gemm_tile(m, k, n, BITS)) {
+  switch (gemm_tile(m, n, BITS)) {
     case GemmTile::k256:
       launch_gemm<BITS, 256, 256, 512, 2>(x, xs, m, k, packed, scales, bias, n, g, y, ys, s);
       break;
@@ -1905,10 +1905,10 @@ bool gemm_rope_shape(int32_t m, int32_t k, int32_t n, int32_t heads, int32_t hea
   if (head_dim != 64 || int64_t(heads) * head_dim != n || m <= EDGERAG_SKINNY_MAX_M ||
       k % kBK != 0)
     return false;
-  if (const int rem = gemm_remainder(m, k, n, 8))
+  if (const int rem = gemm_remainder(m, n, 8))
     return gemm_rope_shape(m - rem, k, n, heads, head_dim) &&
            stream_rope_shape(rem, k, n, heads, head_dim);
-  return gemm_tile(m, k, n, 8) != GemmTile::k64;
+  return gemm_tile(m, n, 8) != GemmTile::k64;
 }
 
 template <int MT, bool NORM = false>
@@ -1961,8 +1961,8 @@ void launch_qlinear_rope(const f16* x, int64_t xs, int32_t m, int32_t k, const u
                          const f16* scales, const f16* bias, int32_t n, const EpiArgs& ea,
                          hipStream_t s) {
   if (!stream_rope_shape(m, k, n, ea.n_q_heads + 2 * ea.n_kv_heads, ea.head_dim)) {
-    const GemmTile tile = gemm_tile(m, k, n, 8);
-    if (const int rem = gemm_remainder(m, k, n, 8)) {
+    const GemmTile tile = gemm_tile(m, n, 8);
+    if (const int rem = gemm_remainder(m, n, 8)) {
       launch_qlinear_rope(x, xs, m - rem, k, packed, scales, bias, n, ea, s);
       const int t0 = m - rem;
       EpiArgs er = ea;

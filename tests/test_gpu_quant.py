@@ -257,9 +257,10 @@ def test_quant_linear_rope_append_fused(device, n_q, n_kv, d, k, with_bias) -> N
 
 
 @pytest.mark.parametrize("n_q,n_kv,k,ms", [
-    (32, 32, 2048, (384, 512, 519, 544)),  # config 5's q/k/v: 128x64 tiles
+    (32, 32, 2048, (384, 512, 519, 544)),  # config 5's q/k/v: 128x64 tiles, 128x128 from M = 519
     (48, 16, 2048, (512, 519)),            # GQA: q / k / v boundaries between workgroups' heads
-    (64, 64, 1024, (200, 512, 519, 544)),  # 128x128 tiles from M = 257; M = 519 streams 7 rows
+    # 128x256 tiles at M = 512 (M = 519 streams 7 rows behind them), else 128x128
+    (64, 64, 1024, (200, 512, 519, 544)),
 ])
 def test_quant_linear_rope_append_tiled_gemm(device, n_q, n_kv, k, ms) -> None:
     """q/k/v projection + RoPE + KV append in the tiled GEMM's epilogue (prefill slices, M > 64,
@@ -314,8 +315,8 @@ def test_quant_linear_rope_append_tiled_gemm(device, n_q, n_kv, k, ms) -> None:
 ])
 def test_quant_linear_swiglu_tiled_gemm(device, k, n, ms) -> None:
     """SwiGLU in the tiled GEMM's epilogue (prefill slices, M > 64, weights whose plain launch
-    takes 128-row tiles: 128x128 for 2048 -> 16384 and 1152 -> 8192 at M = 512, 128x64 for
-    2048 -> 6144): bit-identical to the projection followed by silu_mul, including M = 519
+    takes 128-row tiles: 128x256 for 2048 -> 16384 and 128x128 for 1152 -> 8192 at
+    M = 512, 128x64 for 2048 -> 6144): bit-identical to the projection followed by silu_mul, including M = 519
     (512 chunk tokens + 7 decode rows: the remainder on the streaming SwiGLU kernel where the
     plain launch streams it too) and M = 544; within the linear tolerance of the oracle."""
     w = _weight(n, k, n + 5 * k)
@@ -702,3 +703,17 @@ def test_gemm_tiles_of_a_round_equal_the_small_ones(device, bits, m, k, n, g, st
         assert kernels.quant_swiglu_fused(m, k, n, bits, g)
         fused = kernels.quant_linear_swiglu(x, packed, scales, bias, k, n, bits, g)
         assert torch.equal(fused, kernels.silu_mul(got, n // 2))
+
+
+@pytest.mark.parametrize("m", [369, 384, 385, 496, 497, 512, 513, 624, 625, 640])
+def test_short_last_rows_of_tiles_equal_whole_ones(device, m) -> None:
+    """INT8 layers on either side of the line between 128x128 tiles for less than a round and 128x64
+    ones (a last row of tiles 16 rows short): the bits of the same rows run 91 to 104 at a time."""
+    k, n = 128, 6144
+    gen = torch.Generator(device=device).manual_seed(m)
+    packed, scales = kernels.quantize(torch.randn(n, k, generator=gen, device=device) * 0.02, 8, k)
+    x = torch.randn(m, k, generator=gen, device=device).half()
+    got = kernels.quant_linear(x, packed, scales, None, k, n, 8, k, split_k=False)
+    rows = [kernels.quant_linear(part, packed, scales, None, k, n, 8, k, split_k=False)
+            for part in x.tensor_split(m // 90)]
+    assert torch.equal(got, torch.cat(rows))
