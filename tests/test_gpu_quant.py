@@ -705,6 +705,23 @@ def test_gemm_tiles_of_a_round_equal_the_small_ones(device, bits, m, k, n, g, st
         assert torch.equal(fused, kernels.silu_mul(got, n // 2))
 
 
+@pytest.mark.parametrize("m,n,step", [(1250, 7100, 125), (1300, 6900, 100), (1110, 8100, 111),
+                                      (2040, 8100, 120)])
+def test_every_tile_of_an_uneven_wide_grid_is_written(device, m, n, step) -> None:
+    """256x256 tiles on grids that end within a group of four tile rows or give some XCDs one tile
+    more than others (28 x 5, 27 x 6, 32 x 5 and 32 x 8 tiles): an output filled with NaN comes back
+    with the bits of the same rows run ``step`` at a time (no remainder for the streaming kernel)."""
+    k = 64
+    gen = torch.Generator(device=device).manual_seed(m + n)
+    packed, scales = kernels.quantize(torch.randn(n, k, generator=gen, device=device) * 0.02, 8, k)
+    x = torch.randn(m, k, generator=gen, device=device).half()
+    out = torch.full((m, n), float("nan"), device=device, dtype=torch.float16)
+    got = kernels.quant_linear(x, packed, scales, None, k, n, 8, k, out=out, split_k=False)
+    rows = [kernels.quant_linear(x[i : i + step], packed, scales, None, k, n, 8, k, split_k=False)
+            for i in range(0, m, step)]
+    assert got.data_ptr() == out.data_ptr() and torch.equal(out, torch.cat(rows))
+
+
 @pytest.mark.parametrize("m", [369, 384, 385, 496, 497, 512, 513, 624, 625, 640])
 def test_short_last_rows_of_tiles_equal_whole_ones(device, m) -> None:
     """INT8 layers on either side of the line between 128x128 tiles for less than a round and 128x64
