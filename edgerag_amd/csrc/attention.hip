@@ -1074,12 +1074,13 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
   // slices beside 24 decodes of up to 7,472 tokens, 707 MB of rows: 0.175 against 0.258 ms on
   // one stream. One 512-token chunk, 128 tiles, beside 7 decodes of 32-256 MB: every prefill
   // iteration of the config-5 serving trace was faster on one stream.) Two kinds of batch gain
-  // nothing beside each other and stay on one stream, us on two / one: fp32, but for
-  // grouped rows in parts of contexts (two 300-token slices, 32/32 heads of 64 beside 12 decodes of
-  // 4,096 tokens 220 / 181, 32/8 of 64 with 48 of 6,000 274 / 246, 16/16 of 128 with 8 of 4,096 155 /
-  // 142; in parts 32/8 of 128 with 24 of 4,096 249 / 274, 32/8 of 64 142 / 141), and bf16 tiles of head_dim 128 beside rows of
-  // the VALU kernel, whose fp32 queries want the registers (32/32 heads, two 512-token slices, 8 of
-  // 4,096 225 / 214, 24 of 1,500 213 / 194; fp16 160 / 209, 174 / 182).
+  // nothing beside each other and stay on one stream, us on two / one: fp32, but for grouped rows
+  // in parts of contexts (two 300-token slices, 32/32 heads of 64 beside 12 decodes of 4,096
+  // tokens 220 / 181, 32/8 of 64 with 48 of 6,000 274 / 246, 16/16 of 128 with 8 of 4,096 155 / 142;
+  // in parts 32/8 of 128 with 24 of 4,096 249 / 274, 32/8 of 64 142 / 141), and bf16 tiles of
+  // head_dim 128 beside rows of the VALU kernel, whose fp32 queries want the registers (32/32
+  // heads, two 512-token slices, 8 of 4,096 225 / 214, 24 of 1,500 213 / 194; fp16 160 / 209,
+  // 174 / 182).
   int64_t max_vecs = 0;  // most query vectors of a row
   for (int r = 0; r < num_reqs; ++r) {
     const int64_t v = (int64_t(query_start_loc[r + 1]) - query_start_loc[r]) * n_rep;
@@ -1176,7 +1177,7 @@ extern "C" int edgerag_attn_plan_ex(const int32_t* query_start_loc, const int32_
   // one workgroup per CU (the rows take the rest of each CU), otherwise at two: kTargetTiles / 2
   // or kTargetTiles items. (Three 512-token slices, 384 tiles, beside 24 decodes: splitting them to
   // 768 items for the larger target measured 0.225 against 0.215 ms per step.) Batches of at most
-  // one tile per CU whose tiles hold p in 32 bits (bf16, or head_dim 128) aim at kTargetTiles / 2
+  // one tile per CU whose tiles hold p in two parts (bf16, or head_dim 128) aim at kTargetTiles / 2
   // as well: the partials of twice the items cost more than the second workgroup per CU gains (512
   // tokens at 3,072 keys: fp16 32/8 heads of 128 65.3 -> 62.0 us, bf16 32/32 of 64 43.3 -> 40.9;
   // bf16 32/8 of 128, slices at 2,048 and 4,096: 139 -> 128 us). So do larger batches at head_dim

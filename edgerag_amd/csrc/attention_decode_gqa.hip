@@ -15,14 +15,17 @@
 //     from the pool straight into a buffer of the wave in LDS (no staging registers) and is read
 //     transposed (ds_read_b64_tr_b16).
 // The next step's K (registers) and V (the other LDS buffer) are in flight while a step is
-// computed; waves do not wait for each other before the merge. Items are run as attn_decode_kernel
+// computed (as compiled, the exit in the middle of the loop and the branches that the block offsets
+// become make a wave wait for some of those K loads early); waves do not wait for each other before
+// the merge. Items are run as attn_decode_kernel
 // runs them: one wave per KV split, or a workgroup whose waves split the item's keys and merge in
 // LDS. A fused append stores the item's new rows to their slots first and reads them back from the
 // pool, unless a slot is not the row's place in the block table (a padded token's negative slot):
 // the item's new rows then come from the caller's rows, key by key after the others.
 //
 // Bound by the K/V stream at large batches (bf16 32/8 heads of 128, 48 requests of 256-8,192
-// tokens, 870 MB: 213 -> 159 us, 4.1 -> 5.5 TB/s), by the chain of one wave's steps in small ones (one
+// tokens, 870 MB, append, rows and merge in a stream of steps: 175.5 -> 156.9 us, 5.5 TB/s; the rows'
+// launch replayed alone from a graph 213 -> 159), by the chain of one wave's steps in small ones (one
 // request of 2,048 tokens 18.0 -> 9.6 us, 32 requests with 9/3 heads of 64 44.8 -> 25.2 us).
 #include "attention_merge.h"
 #include "attention_plan.h"

@@ -24,16 +24,19 @@
 //     bits of p in bf16 (error 2^-16 of it), 22 in fp16 (2^-22, down to the floor beside
 //     kTopLog2), where the output is rounded to 8 and 11.
 // A wave computes the scores of tile i + 1 while it exponentiates those of tile i, and scales and
-// reduces them while it accumulates P V of tile i: matrix and VALU work that do not depend on each
-// other alternate in the instruction stream. What bounds a tile now is instruction issue: at two
-// waves per SIMD a wave's 64-key tile takes ~1,600 cycles at head_dim 64 (130 VALU instructions of
-// ~4 cycles, 32 of them exponentials, and 16 MFMAs of 32 cycles) and ~3,000 at 128 (48 MFMAs);
-// taking out the loads, the exponentials or the P V products each gains about 10%.
+// reduces them while it accumulates P V of tile i: at head_dim 64, matrix and VALU work that do not
+// depend on each other alternate in the instruction stream, and issue bounds a tile: at two waves
+// per SIMD a wave's 64-key tile takes ~1,600 cycles (130 VALU instructions of ~4 cycles, 32 of them
+// exponentials, and 16 MFMAs of 32 cycles); taking out the loads, the exponentials or the P V
+// products each gains about 10%. At head_dim 128 (48 MFMAs) the 256 registers do not hold it all: 15
+// are spilled, and in every second tile their reloads share the load counter with the prefetch just
+// issued, so the wave waits for it; a tile takes ~6,500 cycles (87 us for items of 32
+// tiles), twice what its instructions need.
 // Measured: bf16, 32/8 heads of 128, two 512-token slices at 2,048 and 4,096 keys beside 7 decodes
-// 4,388 us on the row kernel -> 123 us; four such slices at 4,096 keys, 129 GFLOP, 195 us (660
-// TFLOP/s). fp16 head_dim 64 against staging through registers with a transposing LDS write:
-// three slices beside 24 decodes 208 -> 206 us, a decoder's prefill iteration (4 layers)
-// 880 -> 864 us.
+// 4,387 us on the row kernel -> 111 us a step in a stream of steps (append, tiles, rows and merge; the
+// tiles 87); four such slices at 4,096 keys, 129 GFLOP, 195 us (660 TFLOP/s). fp16 head_dim 64 against
+// staging through registers with a transposing LDS write: a decoder's prefill iteration (4
+// layers) 880 -> 864 us.
 // The output is O / l or, for split items, fp32 partials merged by attn_combine_kernel.
 #include "attention_plan.h"
 
@@ -212,7 +215,8 @@ __device__ __forceinline__ void fetch_tile(Slice s, char* dst, int lane, int lke
   }
 }
 
-// Two waves per SIMD: the register budget (256 per lane) keeps two tiles' scores, O and Q in VGPRs.
+// Two waves per SIMD: the register budget (256 per lane) keeps two tiles' scores, O and Q in VGPRs,
+// at head_dim 128 but for 15 of them.
 template <typename T, int D>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_prefill_mfma_kernel(

@@ -15,10 +15,11 @@
 //   Only the lane-to-k assignment inside a k-step differs from textbook order, identically for
 //   both operands: INT4 nibbles decode to the k order (0,4,1,5,2,6,3,7), so the activations are
 //   permuted the same way in registers.
-// * qlinear_gemm_kernel (M > 64, prefill slices): MFMA-bound. A workgroup of 256 (or, of
-//   the 128x256 and 256x256 tiles, 512) threads computes a BN x BM tile of y^T through v_mfma_f32_32x32x16_f16; per 64-k step it stages the dequantised
-//   weights and the activations in double-buffered, XOR-swizzled LDS, loading the next steps'
-//   bytes from global memory while the current one is computed. With a workspace
+// * qlinear_gemm_kernel (M > 64, prefill slices): MFMA-bound. A workgroup of 256 threads
+//   (512 for the 128x256 and 256x256 tiles) computes a BN x BM tile of y^T through
+//   v_mfma_f32_32x32x16_f16; per 64-k step it stages the dequantised weights and the activations in
+//   double-buffered, XOR-swizzled LDS, loading the next steps' bytes from global memory while the
+//   current one is computed. With a workspace
 //   (edgerag_quant_linear_ws) it also takes decode batches past the streaming GEMV's crossover,
 //   and splits K over the workgroups when the 64x64 tiles alone would leave CUs idle
 //   (qlinear_split_reduce_kernel adds the k ranges' partial tiles in order).
@@ -1616,8 +1617,9 @@ void dispatch_stream_residual(const f16* x, int64_t xs, int32_t m, int32_t k,
 // 256x256 tiles (512 threads, two waves per SIMD; an operand read from LDS feeds twice the MFMAs of
 // a 128x128 tile) where they are faster than 128x128. Modelled in rounds over the 256 CUs: a full
 // round of 256x256 tiles takes 3.3 rounds of 128x128 ones, a last, partial round 2.4 to 3.3.
-// Measured, 128x128 / 256x256 tiles, us: INT8 2,048 rows 2048 -> 16384 184 / 156, 2048 -> 8192 91 /
-// 76, 1,024 rows 2048 -> 16384 93 / 77, 512 rows 48 / 61; INT4 2,048 rows 4608 -> 4608 157 / 131.
+// Measured, 128x128 / 256x256 tiles, us a call in a stream of calls, weights from memory: INT8 2,048
+// rows 2048 -> 16384 170 / 141, 2048 -> 8192 84 / 72, 1,024 rows 2048 -> 16384 85 / 72; 512 rows 48 / 61;
+// INT4 2,048 rows 4608 -> 4608 153 / 129.
 // Sums run in the same order: the same bits.
 bool gemm_tiles_256(int32_t m, int32_t n) {
   const int64_t t256 = int64_t((n + 255) / 256) * ((m + 255) / 256);

@@ -207,8 +207,10 @@ int edgerag_paged_attention(const int32_t* plan_host, const int32_t* plan_dev, i
  * same results. When every work item of the plan is a decode row on the fast decode kernel (the
  * usual decode batch) and the new rows are in the pool dtype and 16-byte aligned, it is one
  * launch: the waves that reach a request's new positions read them from new_key / new_value and
- * write them to the pools at their slots; the attention treats a token's new K/V as sitting at
- * its position in the block table, as slot_mapping does when built from the tables. Otherwise
+ * write them to the pools at their slots (rows of several query vectors may read them back from
+ * there where the slot is the position's place in the block table); the attention treats a token's
+ * new K/V as sitting at its position in the block table, as slot_mapping does when built from the
+ * tables, also where a token's slot is negative or elsewhere. Otherwise
  * (prefill tiles in the batch, other layouts) it enqueues the two launches.
  *
  * Replaces PagedKVCache._write followed by fused_paged_attention for a decode step

@@ -398,9 +398,9 @@ def test_fp16_prefill_chunk_edges(device, c, past) -> None:
                                      (torch.float32, 128)])
 @pytest.mark.parametrize("n_q,n_kv", [(4, 4), (6, 2), (8, 2)])
 def test_wide_prefill_tile_edges(device, dtype, d, n_q, n_kv) -> None:
-    """The tiles that hold p in 32 bits (the fp32 ones too): one token past the row limit, one short of and past a
-    128-row tile, chunks below, at and past a 64-key tile, odd prefixes and a split context, all
-    in one batch whose unwritten pool rows are NaN, against the float64 softmax. The error is the
+    """The tiles that hold p in two parts, and the fp32 ones: one token past the row limit, one short
+    of and past a 128-row tile, chunks below, at and past a 64-key tile, odd prefixes and a split
+    context, all in one batch whose unwritten pool rows are NaN, against the float64 softmax. The error is the
     rounding of the output (2^-8 relative for bf16, 2^-11 for fp16) plus that of hi + lo
     (2^-16, 2^-22)."""
     rep = n_q // n_kv
@@ -424,10 +424,10 @@ def test_wide_prefill_tile_edges(device, dtype, d, n_q, n_kv) -> None:
 
 @pytest.mark.parametrize("dtype,d,reqs", [(torch.float16, 128, 1), (torch.float32, 64, 1),
                                           (torch.float32, 128, 12)])
-@pytest.mark.parametrize("bs", [1, 4, 32, 128])
+@pytest.mark.parametrize("bs", [1, 4, 24, 32, 128])
 def test_wide_prefill_tiles_at_other_block_sizes(device, dtype, d, reqs, bs) -> None:
     """Blocks smaller and larger than a 64-key tile (the row kernel takes blocks of less than 4 in
-    fp16), a bad block id in the table's tail, and enough requests for 32-row fp32 tiles."""
+    fp16 and those that are no power of two), a bad block id in the table's tail, and enough requests for 32-row fp32 tiles."""
     g = seeded(bs + d)
     c, L, h = 70, 333, 2
     nb = -(-L // bs)

@@ -316,9 +316,9 @@ def test_quant_linear_rope_append_tiled_gemm(device, n_q, n_kv, k, ms) -> None:
 def test_quant_linear_swiglu_tiled_gemm(device, k, n, ms) -> None:
     """SwiGLU in the tiled GEMM's epilogue (prefill slices, M > 64, weights whose plain launch
     takes 128-row tiles: 128x256 for 2048 -> 16384 and 128x128 for 1152 -> 8192 at
-    M = 512, 128x64 for 2048 -> 6144): bit-identical to the projection followed by silu_mul, including M = 519
-    (512 chunk tokens + 7 decode rows: the remainder on the streaming SwiGLU kernel where the
-    plain launch streams it too) and M = 544; within the linear tolerance of the oracle."""
+    M = 512, 128x64 for 2048 -> 6144): bit-identical to the projection followed by silu_mul,
+    including M = 519 (512 chunk tokens + 7 decode rows: the remainder on the streaming SwiGLU
+    kernel where the plain launch streams it too) and M = 544; within the linear tolerance of the oracle."""
     w = _weight(n, k, n + 5 * k)
     cfg = oq.QuantConfig(k, 8)
     packed, scales = oq.quantize_for_layer(w, cfg)
