@@ -427,7 +427,8 @@ def test_wide_prefill_tile_edges(device, dtype, d, n_q, n_kv) -> None:
 @pytest.mark.parametrize("bs", [1, 4, 24, 32, 128])
 def test_wide_prefill_tiles_at_other_block_sizes(device, dtype, d, reqs, bs) -> None:
     """Blocks smaller and larger than a 64-key tile (the row kernel takes blocks of less than 4 in
-    fp16 and those that are no power of two), a bad block id in the table's tail, and enough requests for 32-row fp32 tiles."""
+    fp16 and those that are no power of two), a bad block id in the table's tail, and enough
+    requests for 32-row fp32 tiles."""
     g = seeded(bs + d)
     c, L, h = 70, 333, 2
     nb = -(-L // bs)
